@@ -66,15 +66,16 @@ struct ien_ctx {
   // to single kernels.
   bool serial_branches = false;
   // Chains of body pairs (conv_pair.hip): an abort word, a failure word, a
-  // count of workgroups done and chain_tiles epoch words; the workgroups of the chain kernel one CU
-  // holds (-1 until asked); the wall-clock ticks (100 MHz) a tile may wait
-  // for a neighbour.
+  // count of workgroups done and chain_tiles epoch words; the workgroups of
+  // each tiling's chain kernel that one CU holds (-1 until asked); the
+  // wall-clock ticks (100 MHz) a tile may wait for a neighbour.
   int *chain_flags = nullptr;
   // Sequence number of the last chain launched on this context, and the
   // highest failed one already reported (chain_status).
   int chain_seq = 0, chain_reported = 0;
   int chain_tiles = 0;
-  int chain_per_cu = -1;
+  static constexpr int CHAIN_TILINGS = 3;
+  int chain_per_cu[CHAIN_TILINGS] = {-1, -1, -1};
   long chain_spin = 100000000;
 };
 
