@@ -16,8 +16,10 @@ struct Lama {
   ien_ctx *ctx = nullptr;
   ien_matrix *first = nullptr, *down[3] = {}, *up[3][4] = {}, *last = nullptr;
   LamaFfc blocks[18][2];
-  ien_fourier *fourier = nullptr;  // for the eighth-scale maps of the current size
-  ien_spectral *spectral_plan = nullptr;  // the fused spectral branch (sides <= 64), else null
+  // For the eighth-scale maps of the current size: the fused spectral branch
+  // (sides <= 128), or the transforms of the unfused one.
+  ien_spectral *spectral_plan = nullptr;
+  ien_fourier *fourier = nullptr;
   size_t pw = 0, ph = 0;           // padded size the maps and the plan are for
   size_t pixels = 0;               // padded pixels the maps hold
   // Full-scale 4-channel input; maps at 1, 1/2, 1/4 (reused by the ups);
@@ -52,17 +54,21 @@ ien_status spectral_front(const ien_spectral *sp, const uint16_t *x, long xs,
                           const ien_matrix *m_in, const ien_matrix *m_f, uint16_t *spectral,
                           float *r, float *u);
 // The front's two launches one at a time: the rows (spectral map and R),
-// then the columns (U).
+// then the columns (U; `z` holds the spectrum of a map over 64 rows, half x
+// (h rounded up to 32) pixels of 384 halves, and is not used otherwise).
 ien_status spectral_rows(const ien_spectral *sp, const uint16_t *x, long xs,
                          const ien_matrix *m_in, uint16_t *spectral, float *r);
 ien_status spectral_columns(const ien_spectral *sp, const ien_matrix *m_f, const float *r,
-                            float *u);
+                            uint16_t *z, float *u);
 // The result (ReLU(out + spectral_out(spectral + irfft(u)))) goes to dst
 // (out when null), with `add` (rows ys apart, or null) added after the
 // rounding and rounded again.
 ien_status spectral_back(const ien_spectral *sp, const ien_matrix *m_out, const uint16_t *spectral,
                          const float *u, uint16_t *out, long ys, uint16_t *dst = nullptr,
                          const uint16_t *add = nullptr);
+// A plan of any map it fits (sides up to 128; ien_spectral_new takes 64).
+bool spectral_fits(size_t height, size_t width);
+ien_status spectral_new(ien_ctx *ctx, size_t height, size_t width, ien_spectral **out);
 size_t spectral_r_floats(const ien_spectral *sp);
 size_t spectral_u_floats(const ien_spectral *sp);
 

@@ -7,10 +7,12 @@
 //   spectral += irfftn(filtered), "ortho"                    fourier.rs:347-403
 //   out       = ReLU(out + spectral spectral_out)            1x1, 192 -> 384, accumulated
 //
-// for maps of at most 64 x 64 (LaMa's eighth scale up to 512 x 512 images).
-// The unfused path (fourier.hip and four products) takes seven dependent
-// launches, each a load -> compute -> store chain of a few microseconds on a
-// map of 1.5 MB; here:
+// for maps of at most 64 x 64 (LaMa's eighth scale up to 512 x 512 images),
+// and in three or four for sides of up to 128 (the wide and tall kernels
+// below: a side over 64 takes its own variant of the launches that hold a
+// whole line of that direction).  The unfused path (fourier.hip and four
+// products) takes seven dependent launches, each a load -> compute -> store
+// chain of a few microseconds on a map of 1.5 MB; here:
 //
 //   front  (one workgroup per map row and 64-channel group): the spectral_in
 //          product for the row's pixels, bias, ReLU, f16 (the spectral map,
@@ -37,8 +39,8 @@
 // hi = f16(v), lo = f16(v - hi) and each table entry likewise, and a product
 // sums hi.hi + lo.hi + hi.lo (|error| about 2^-22 of the terms): the split is
 // one more stretch of the reduction (K) dimension.  f32 intermediates are
-// scaled by powers of two before the split (R by 2^-6, U by 2^-8, undone in
-// the tables) so that no half overflows.  The rounding points are those of
+// scaled by powers of two before the split (R by 2^-6, or 2^-7 for rows over
+// 64, U by 2^-8, undone in the tables) so that no half overflows.  The rounding points are those of
 // the unfused path: the spectral map, the spectrum and the filtered spectrum
 // in f16, the transforms' sums in f32.
 //
@@ -61,8 +63,11 @@ namespace {
 constexpr int GLOBAL_C = 384;  // the FFC's global channels (the product's input)
 constexpr int SPEC = 192;      // spectral channels
 constexpr int SPEC2 = 384;     // spectrum values per pixel: re x 192 | im x 192
-constexpr int MAX_SIDE = 64;
-constexpr float RSCALE = 1.0f / 64, USCALE = 1.0f / 256;
+constexpr int MAX_SIDE = 64;   // of the public plans, and of the kernels without a wide or tall variant
+constexpr int LONG_SIDE = 128;  // of the wide and tall kernels
+constexpr float USCALE = 1.0f / 256;
+// R's scale before the split: a row sums up to w f16 values.
+constexpr float r_scale(int w) { return w <= MAX_SIDE ? 1.0f / 64 : 1.0f / 128; }
 constexpr int COLUMN_GROUPS = 6;  // 32 channels a columns workgroup
 constexpr int BACK_GROUPS = 3;    // 128 output channels a back workgroup
 
@@ -207,6 +212,7 @@ struct ColumnArgs {
   int kb_f;
   const float *b_f;
   float *u;  // [h][half][384]
+  float rscale;
 };
 
 constexpr int RP = MAX_SIDE + 8;                        // halves per transposed R row
@@ -285,7 +291,7 @@ __global__ __launch_bounds__(512) void k_spectral_columns(ColumnArgs p) {
         for (int cc = 0; cc < 4; cc++) {
           float f[8];
 #pragma unroll
-          for (int j = 0; j < 8; j++) f[j] = v[b][j][cc] * RSCALE;
+          for (int j = 0; j < 8; j++) f[j] = v[b][j][cc] * p.rscale;
           half8 vh, vl;
           split8(f, vh, vl);
           const int row = part * SPEC + 4 * c4 + cc;
@@ -616,6 +622,408 @@ __global__ __launch_bounds__(256) void k_spectral_back(BackArgs p) {
   }
 }
 
+// ---- lines of 65 .. 128 points ----------------------------------------------
+//
+// LaMa's maps of images over 512 pixels a side.  On 125 x 85 (1000 x 680
+// images) the unfused chain took 113 us of launches, 80 of them in four line
+// passes on f32 MFMA (1/16 of the f16 rate) with a table load per step;
+// these four take 15.5 (front), 14.5 and 14.9 (columns) and 20 us (back),
+// beside the convolutions' streams.  What bounds them is latency: each is
+// one load -> split -> product -> store chain a CU, at a round or less of
+// workgroups.
+
+// front over rows of 65 .. 128 pixels: eight waves, one 32-channel x 32-pixel
+// block of the product each, then one 32 x 32 block of the row transform
+// each.  A workgroup holds its row (96 KiB) and its group's weights (48 KiB),
+// one a CU; the table fragments stay in registers and the transposed
+// spectral row takes the pixels' place after the product.
+constexpr int SPW = LONG_SIDE + 8;
+constexpr int FW_W = 96 * 1024, FRONT_WIDE_LDS = FW_W + 48 * 1024;
+
+// The row and part of block b: parts of one row on one XCD (block b runs on
+// XCD b % 8), so that what they share comes from that XCD's L2.
+__device__ __forceinline__ void row_part(int b, int parts, int &row, int &part) {
+  const int slot = b >> 3;
+  row = (b & 7) + 8 * (slot / parts);
+  part = slot % parts;
+}
+
+__global__ __launch_bounds__(512) void k_spectral_front_wide(FrontArgs p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[FRONT_WIDE_LDS];
+  uint16_t *st = (uint16_t *)lds;  // after the product
+  int y, g;
+  row_part(blockIdx.x, SPEC / 64, y, g);
+  if (y >= p.h) return;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 31, hi = lane >> 5;
+  constexpr int KS = GLOBAL_C / 16, TS = 2 * LONG_SIDE / 16;
+  const int ks_t = p.xp / 8;
+  {
+    const uint16_t *row = p.x + (long)y * p.w * p.xs;
+    for (int f = wave; f * 64 < 48 * p.w; f += 8) {
+      const int q = 64 * f + lane, x = q / 48, c = (q - 48 * x) ^ (x & 15);
+      dma16(row + (long)min(x, p.w - 1) * p.xs + 8 * c, lds + f * 1024);
+    }
+    const uint16_t *wg = p.w_in + (long)(2 * g) * p.kb_in * 512 + lane * 8;
+    for (int f = wave; f < 2 * KS; f += 8) {
+      const int nblk = f / KS, ks = f - nblk * KS;
+      dma16(wg + ((long)nblk * p.kb_in + ks) * 512, lds + FW_W + f * 1024);
+    }
+  }
+  const int blk = wave & 1, line = wave >> 1;  // channel block; pixel block, then R's row block
+  float4v bias[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) bias[q] = *(const float4v *)(p.b_in + 64 * g + blk * 32 + 8 * q + 4 * hi);
+  half8 tf[TS];
+  {
+    const uint16_t *tb = p.tf + (long)min(line, p.mb - 1) * ks_t * 512 + lane * 8;
+#pragma unroll
+    for (int i = 0; i < TS; i++) tf[i] = ld8(tb + min(i, ks_t - 1) * 512);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the direct-to-LDS loads have landed
+  __syncthreads();
+  const int x = line * 32 + col;
+  floatx16 acc = {};
+  if (line * 32 < p.w) {
+    const int sx = x & 15;
+    const unsigned char *wa = lds + FW_W + blk * KS * 1024 + lane * 16;
+    const unsigned char *xa = lds + x * 768;
+#pragma unroll
+    for (int i = 0; i < KS; i++)
+      acc = mfma16(*(const half8 *)(wa + i * 1024), *(const half8 *)(xa + (((2 * i + hi) ^ sx) << 4)), acc);
+  }
+  __syncthreads();  // every wave is done with the pixels
+  if (x < p.xp) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int n0 = blk * 32 + 8 * q + 4 * hi;
+      uint16_t *sr = p.s + ((long)y * SPEC + 64 * g + n0) * p.w + x;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const uint16_t v = x < p.w ? f2h(fmaxf(acc[4 * q + j] + bias[q][j], 0.0f)) : (uint16_t)0;
+        st[(n0 + j) * SPW + x] = v;
+        if (x < p.w) sr[(long)j * p.w] = v;
+      }
+    }
+  }
+  __syncthreads();
+  if (line < p.mb) {
+    const int c = blk * 32 + col;
+    floatx16 d = {};
+#pragma unroll
+    for (int i = 0; i < TS; i++)
+      if (i < ks_t) d = mfma16(tf[i], ld8(st + c * SPW + (16 * i + 8 * hi) % p.xp), d);
+    float *out = p.r + (long)y * p.w * SPEC + 64 * g + c;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int m = line * 32 + 8 * (r >> 2) + 4 * hi + (r & 3);
+      if (m < p.w) out[(long)m * SPEC] = d[r];
+    }
+  }
+}
+
+// columns over 65 .. 128 rows, in two launches (a column of all channels
+// would not fit a CU, and every group would transform it again): the column
+// transform of 32 channels a workgroup into the f16 spectrum, then the
+// fourier product of 32 real and 32 imaginary output channels and their
+// inverse columns.  The spectrum lies in the product's A fragments,
+// z[k][ky / 32][c' / 16], so that a wave reads it a KiB at a time.
+constexpr int TALL_STEPS = LONG_SIDE / 16;
+constexpr int ZK = SPEC2 / 16;  // 16-deep steps of the product
+
+struct TallArgs {
+  const float *r;
+  int h, w, half, yp, nba, kyb;  // kyb: 32-blocks of h
+  float rscale;
+  const uint16_t *ta, *tc;  // as ColumnArgs
+  const uint16_t *wf;
+  int kb_f;
+  const float *b_f;
+  uint16_t *z;
+  float *u;
+};
+
+__global__ __launch_bounds__(512, 4) void k_spectral_tall(TallArgs p) {
+  // A fragments of R, [hi | lo][part][y step], written once by the wave
+  // that loads the step's rows.
+  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * TALL_STEPS * 1024];
+  int k, g;
+  row_part(blockIdx.x, COLUMN_GROUPS, k, g);
+  if (k >= p.half) return;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 31, hi = lane >> 5;
+  const int ysteps = p.yp / 16, ks2 = 2 * ysteps;
+  const uint16_t *tb = p.ta + (long)min(wave, p.nba - 1) * 2 * ks2 * 512 + lane * 8;
+  half8 thi[TALL_STEPS], tlo[TALL_STEPS];
+#pragma unroll
+  for (int ys = 0; ys < TALL_STEPS; ys++) {
+    thi[ys] = ld8(tb + min(ys, ysteps - 1) * 512);
+    tlo[ys] = ld8(tb + (ks2 + min(ys, ysteps - 1)) * 512);
+  }
+  if (wave < ysteps) {
+    const int mim = (k >= 1 && k <= p.w - p.half) ? p.half + k - 1 : -1;
+    float v[2][8];
+#pragma unroll
+    for (int part = 0; part < 2; part++) {
+      const int m = part ? mim : k, y0 = 16 * wave + 8 * hi;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const bool ok = m >= 0 && y0 + j < p.h;
+        v[part][j] = p.r[ok ? ((y0 + j) * p.w + m) * SPEC + 32 * g + col : 0];
+        if (!ok) v[part][j] = 0.0f;
+      }
+    }
+#pragma unroll
+    for (int part = 0; part < 2; part++) {
+#pragma unroll
+      for (int j = 0; j < 8; j++) v[part][j] *= p.rscale;
+      half8 vh, vl;
+      split8(v[part], vh, vl);
+      unsigned char *at = lds + (part * TALL_STEPS + wave) * 1024 + lane * 16;
+      *(half8 *)at = vh;
+      *(half8 *)(at + 2 * TALL_STEPS * 1024) = vl;
+    }
+  }
+  __syncthreads();
+  if (wave >= p.nba) return;
+  floatx16 acc = {};
+#pragma unroll
+  for (int part = 0; part < 2; part++)
+#pragma unroll
+    for (int ys = 0; ys < TALL_STEPS; ys++) {
+      if (ys < ysteps) {
+        const unsigned char *at = lds + (part * TALL_STEPS + ys) * 1024 + lane * 16;
+        const half8 ah = *(const half8 *)at, al = *(const half8 *)(at + 2 * TALL_STEPS * 1024);
+        acc = mfma16(ah, thi[ys], acc);
+        acc = mfma16(al, thi[ys], acc);
+        acc = mfma16(ah, tlo[ys], acc);
+        if (part == 0) {  // the imaginary part's fragments, over the real part's
+          thi[ys] = ld8(tb + (ysteps + ys) * 512);
+          tlo[ys] = ld8(tb + (ks2 + ysteps + ys) * 512);
+        }
+      }
+    }
+  const int n = wave * 32 + col;
+  if (n < 2 * p.h) {
+    const int pp = n >= p.h, ky = n - pp * p.h;
+    uint16_t *zb = p.z + ((long)(k * p.kyb + (ky >> 5)) * ZK + (pp * SPEC + 32 * g) / 16) * 512 +
+                   (ky & 31) * 8 + 4 * hi;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      st4h(zb + (q >> 1) * 512 + (q & 1) * 256, acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+  }
+}
+
+// LDS: the group's fourier fragments [part][k step], later the inverse
+// columns' outputs [2h][US_P] f32; the filtered spectrum [2 x 32][SPW].
+constexpr int TB_PT = 2 * ZK * 1024, TALL_BACK_LDS = TB_PT + 64 * SPW * 2;
+static_assert(2 * LONG_SIDE * US_P * 4 <= TB_PT, "staged U over the fragments");
+
+__global__ __launch_bounds__(512, 4) void k_spectral_tall_back(TallArgs p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[TALL_BACK_LDS];
+  uint16_t *pt = (uint16_t *)(lds + TB_PT);
+  float *ustage = (float *)lds;
+  int k, g;
+  row_part(blockIdx.x, COLUMN_GROUPS, k, g);
+  if (k >= p.half) return;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 31, hi = lane >> 5;
+  const int h = p.h, ysteps = p.yp / 16, ks2 = 2 * ysteps;
+  constexpr int CG = SPEC / COLUMN_GROUPS, BATCH = ZK / 2;
+  const int pb = wave >> 1, part = wave & 1;  // the product's block of rows, and part
+  for (int f = wave; f < 2 * ZK; f += 8) {
+    const int fp = f / ZK, i = f - fp * ZK;
+    dma16(p.wf + ((long)((fp * SPEC + CG * g) / 32) * p.kb_f + i) * 512 + lane * 8, lds + f * 1024);
+  }
+  const float bias = p.b_f[part * SPEC + CG * g + col];
+  const uint16_t *zb = p.z + (long)(k * p.kyb + min(pb, p.kyb - 1)) * ZK * 512 + lane * 8;
+  half8 za[BATCH];
+#pragma unroll
+  for (int i = 0; i < BATCH; i++) za[i] = ld8(zb + i * 512);
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the direct-to-LDS loads have landed
+  __syncthreads();
+  if (pb < p.kyb) {
+    const unsigned char *wb = lds + part * ZK * 1024 + lane * 16;
+    floatx16 d = {};
+#pragma unroll
+    for (int i = 0; i < ZK; i++) {
+      d = mfma16(za[i % BATCH], *(const half8 *)(wb + i * 1024), d);
+      if (i < BATCH) za[i] = ld8(zb + (BATCH + i) * 512);
+    }
+    // (Rows past h of the last block were never written: zero here.)
+    uint16_t *dst = pt + (part * CG + col) * SPW;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int ky0 = pb * 32 + 8 * q + 4 * hi;
+      if (ky0 < p.yp) {
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = ky0 + j < h ? fmaxf(d[4 * q + j] + bias, 0.0f) : 0.0f;
+        st4h(dst + ky0, v[0], v[1], v[2], v[3]);
+      }
+    }
+  }
+  const uint16_t *tb = p.tc + (long)min(wave, p.nba - 1) * 2 * ks2 * 512 + lane * 8;
+  half8 thi[TALL_STEPS], tlo[TALL_STEPS];
+#pragma unroll
+  for (int ys = 0; ys < TALL_STEPS; ys++) {
+    thi[ys] = ld8(tb + min(ys, ysteps - 1) * 512);
+    tlo[ys] = ld8(tb + (ks2 + min(ys, ysteps - 1)) * 512);
+  }
+  __syncthreads();
+  if (wave < p.nba) {
+    floatx16 d = {};
+#pragma unroll
+    for (int fp = 0; fp < 2; fp++)
+#pragma unroll
+      for (int ys = 0; ys < TALL_STEPS; ys++) {
+        if (ys < ysteps) {
+          const half8 a = ld8(pt + (fp * CG + col) * SPW + ys * 16 + 8 * hi);
+          d = mfma16(a, thi[ys], d);
+          d = mfma16(a, tlo[ys], d);
+          if (fp == 0) {
+            thi[ys] = ld8(tb + (ysteps + ys) * 512);
+            tlo[ys] = ld8(tb + (ks2 + ysteps + ys) * 512);
+          }
+        }
+      }
+    const int n = wave * 32 + col;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      *(float4v *)(ustage + n * US_P + 8 * q + 4 * hi) =
+          float4v{d[4 * q], d[4 * q + 1], d[4 * q + 2], d[4 * q + 3]};
+  }
+  __syncthreads();
+  for (int q = tid; q < 2 * h * 8; q += 512) {
+    const int n = q >> 3, c4 = q & 7;
+    const int pp = n >= h, yy = n - pp * h;
+    *(float4v *)(p.u + ((yy * p.half + k) * SPEC2 + pp * SPEC + CG * g + 4 * c4)) =
+        *(const float4v *)(ustage + n * US_P + 4 * c4);
+  }
+}
+
+// back over rows of 65 .. 128 pixels: a workgroup of six waves takes 32 of
+// a row's pixels.  Wave w's inverse rows are those of channels 32 w ..: their
+// U goes straight into A fragments (a lane's eight columns of one channel,
+// each read 32 consecutive channels a half wave); then two 32-channel blocks
+// of the spectral_out product over all 192.  Splitting the row by pixels
+// reads U once a block but computes nothing twice.
+constexpr int BACK_WIDE_WAVES = SPEC / 32, OBW = SPEC2 + 8;
+
+// (Three waves a SIMD, so that two workgroups share a CU: 125 x 85 makes 340.)
+__global__ __launch_bounds__(64 * BACK_WIDE_WAVES, 3) void k_spectral_back_wide(BackArgs p) {
+  __shared__ __attribute__((aligned(16))) uint16_t s2[32 * S2P], ob[32 * OBW];
+  int y, xb;
+  row_part(blockIdx.x, p.nbx, y, xb);
+  if (y >= p.h) return;
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, hi = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = p.w, msteps = p.mp / 16, x0 = 32 * xb, xc = min(x0 + col, w - 1);
+  constexpr int MS = LONG_SIDE / 16, KO = SPEC / 16, ITEMS = 32 * SPEC2 / 8 / (64 * BACK_WIDE_WAVES);
+  // The cross output, 16-byte items; U.
+  const long orow = ((long)y * w + x0) * p.ys;
+  u32x4 old[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; i++) {
+    const int q = tid + 64 * BACK_WIDE_WAVES * i, x = min(q / 48, w - 1 - x0);
+    old[i] = *(const u32x4 *)(p.out + orow + (long)x * p.ys + 8 * (q % 48));
+  }
+  const uint16_t *tb = p.tr + (long)xb * 2 * msteps * 512 + lane * 8;
+  const float *ub = p.u + (long)y * p.half * SPEC2 + 32 * wave;
+  floatx16 acc = {};
+#pragma unroll
+  for (int m4 = 0; m4 < MS; m4 += 4) {  // four steps' loads together
+    float f[4][8];
+    half8 thi[4], tlo[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int ms = min(m4 + i, msteps - 1);
+      thi[i] = ld8(tb + ms * 512);
+      tlo[i] = ld8(tb + (msteps + ms) * 512);
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const int m = 16 * (m4 + i) + 8 * hi + j;
+        const bool ok = m < w;
+        const int at = m >= p.half ? (m - p.half + 1) * SPEC2 + SPEC : m * SPEC2;
+        f[i][j] = ub[(unsigned)((ok ? at : 0) + col)];
+        if (!ok) f[i][j] = 0.0f;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      if (m4 + i < msteps) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) f[i][j] *= USCALE;
+        half8 ah, al;
+        split8(f[i], ah, al);
+        acc = mfma16(ah, thi[i], acc);
+        acc = mfma16(al, thi[i], acc);
+        acc = mfma16(ah, tlo[i], acc);
+      }
+    }
+  }
+  uint16_t sv[16];
+  const uint16_t *sc = p.s + ((long)y * SPEC + 32 * wave) * w;
+#pragma unroll
+  for (int r = 0; r < 16; r++) sv[r] = sc[(unsigned)((8 * (r >> 2) + 4 * hi + (r & 3)) * w + xc)];
+  // The first block's weights, requested before the results go to LDS (and
+  // not moved up among U's registers, which would spill).
+  __builtin_amdgcn_sched_barrier(0);
+  const uint16_t *wb = p.wo + (long)wave * p.kb_o * 512;
+  half8 wo[KO];
+#pragma unroll
+  for (int i = 0; i < KO; i++) wo[i] = ld8(wb + i * 512 + lane * 8);
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    st4h(s2 + col * S2P + 32 * wave + 8 * q + 4 * hi, acc[4 * q] + h2f(sv[4 * q]),
+         acc[4 * q + 1] + h2f(sv[4 * q + 1]), acc[4 * q + 2] + h2f(sv[4 * q + 2]),
+         acc[4 * q + 3] + h2f(sv[4 * q + 3]));
+#pragma unroll
+  for (int i = 0; i < ITEMS; i++) {
+    const int q = tid + 64 * BACK_WIDE_WAVES * i;
+    *(u32x4 *)(ob + (q / 48) * OBW + 8 * (q % 48)) = old[i];
+  }
+  if (p.add) {
+#pragma unroll
+    for (int i = 0; i < ITEMS; i++) {
+      const int q = tid + 64 * BACK_WIDE_WAVES * i, x = min(q / 48, w - 1 - x0);
+      old[i] = *(const u32x4 *)(p.add + orow + (long)x * p.ys + 8 * (q % 48));
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    floatx16 d = {};
+#pragma unroll
+    for (int i = 0; i < KO; i++) {
+      d = mfma16(wo[i], ld8(s2 + col * S2P + 16 * i + 8 * hi), d);
+      if (j == 0) wo[i] = ld8(wb + ((long)BACK_WIDE_WAVES * p.kb_o + i) * 512 + lane * 8);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      uint16_t *e = ob + col * OBW + (wave + BACK_WIDE_WAVES * j) * 32 + 8 * q + 4 * hi;
+      const uint2 ov = *(const uint2 *)e;
+      st4h(e, fmaxf(h2f((uint16_t)ov.x) + d[4 * q], 0.0f),
+           fmaxf(h2f((uint16_t)(ov.x >> 16)) + d[4 * q + 1], 0.0f),
+           fmaxf(h2f((uint16_t)ov.y) + d[4 * q + 2], 0.0f),
+           fmaxf(h2f((uint16_t)(ov.y >> 16)) + d[4 * q + 3], 0.0f));
+    }
+  }
+  __syncthreads();
+  uint16_t *og = p.dst + orow;
+#pragma unroll
+  for (int i = 0; i < ITEMS; i++) {
+    const int q = tid + 64 * BACK_WIDE_WAVES * i, x = q / 48;
+    if (x0 + x >= w) continue;
+    uint16_t o[8];
+    *(u32x4 *)o = *(const u32x4 *)(ob + x * OBW + 8 * (q % 48));
+    if (p.add) {
+      uint16_t a[8];
+      *(u32x4 *)a = old[i];
+#pragma unroll
+      for (int e = 0; e < 8; e++) o[e] = f2h(h2f(o[e]) + h2f(a[e]));
+    }
+    *(u32x4 *)(og + (long)x * p.ys + 8 * (q % 48)) = *(const u32x4 *)o;
+  }
+}
+
 // ---- host: the tables ------------------------------------------------------
 
 float half_bits_to_float(uint16_t h) {
@@ -655,6 +1063,17 @@ std::vector<uint16_t> operand(int blocks, int ksteps, F value) {
   return out;
 }
 
+// cos and sin of 2 pi j / n, j < n, in turn.
+std::vector<double> circle(int n) {
+  std::vector<double> t(2 * (size_t)n);
+  for (int j = 0; j < n; j++) {
+    const double a = 6.283185307179586476925 * (double)j / n;
+    t[2 * j] = std::cos(a);
+    t[2 * j + 1] = std::sin(a);
+  }
+  return t;
+}
+
 int up16(int n) { return (n + 15) / 16 * 16; }
 
 }  // namespace
@@ -680,18 +1099,32 @@ ien_status spectral_rows(const ien_spectral *sp, const uint16_t *x, long xs,
   ien_ctx *ctx = sp->ctx;
   FrontArgs a{x, (int)xs, sp->h, sp->w, sp->xp, sp->mb, m_in->d_packed, m_in->kb, m_in->d_bias,
               sp->d_tf, spectral, r};
-  hipLaunchKernelGGL(k_spectral_front, dim3((unsigned)sp->h, SPEC / 64), dim3(256), 0, ctx->stream,
-                     a);
+  if (sp->w > MAX_SIDE)
+    hipLaunchKernelGGL(k_spectral_front_wide, dim3(8u * (SPEC / 64) * (unsigned)((sp->h + 7) / 8)),
+                       dim3(512), 0, ctx->stream, a);
+  else
+    hipLaunchKernelGGL(k_spectral_front, dim3((unsigned)sp->h, SPEC / 64), dim3(256), 0, ctx->stream,
+                       a);
   IEN_HIP(hipGetLastError());
   return IEN_OK;
 }
 
 ien_status spectral_columns(const ien_spectral *sp, const ien_matrix *m_f, const float *r,
-                            float *u) {
+                            uint16_t *z, float *u) {
   ien_ctx *ctx = sp->ctx;
-  ColumnArgs c{r, sp->h, sp->w, sp->half, sp->yp, sp->nba, sp->d_ta, sp->d_tc, m_f->d_packed,
-               m_f->kb, m_f->d_bias, u};
   const unsigned column_blocks = 8u * COLUMN_GROUPS * (unsigned)((sp->half + 7) / 8);
+  if (sp->h > MAX_SIDE) {
+    IEN_CHECK(z && ((uintptr_t)z & 15) == 0, IEN_ERR_INPUT, "spectrum buffer of a tall map");
+    TallArgs t{r, sp->h, sp->w, sp->half, sp->yp, sp->nba, (sp->h + 31) / 32, r_scale(sp->w),
+               sp->d_ta, sp->d_tc, m_f->d_packed, m_f->kb, m_f->d_bias, z, u};
+    hipLaunchKernelGGL(k_spectral_tall, dim3(column_blocks), dim3(512), 0, ctx->stream, t);
+    IEN_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_spectral_tall_back, dim3(column_blocks), dim3(512), 0, ctx->stream, t);
+    IEN_HIP(hipGetLastError());
+    return IEN_OK;
+  }
+  ColumnArgs c{r, sp->h, sp->w, sp->half, sp->yp, sp->nba, sp->d_ta, sp->d_tc, m_f->d_packed,
+               m_f->kb, m_f->d_bias, u, r_scale(sp->w)};
   hipLaunchKernelGGL(k_spectral_columns, dim3(column_blocks), dim3(512), 0, ctx->stream, c);
   IEN_HIP(hipGetLastError());
   return IEN_OK;
@@ -701,7 +1134,7 @@ ien_status spectral_front(const ien_spectral *sp, const uint16_t *x, long xs,
                           const ien_matrix *m_in, const ien_matrix *m_f, uint16_t *spectral,
                           float *r, float *u) {
   const ien_status st = spectral_rows(sp, x, xs, m_in, spectral, r);
-  return st == IEN_OK ? spectral_columns(sp, m_f, r, u) : st;
+  return st == IEN_OK ? spectral_columns(sp, m_f, r, nullptr, u) : st;
 }
 
 ien_status spectral_back(const ien_spectral *sp, const ien_matrix *m_out, const uint16_t *spectral,
@@ -712,24 +1145,26 @@ ien_status spectral_back(const ien_spectral *sp, const ien_matrix *m_out, const 
             "spectral output and added map 16-byte aligned");
   BackArgs b{u, sp->h, sp->w, sp->half, sp->xp, sp->nbx, sp->d_tr, spectral, m_out->d_packed,
              m_out->kb, out, (int)ys, dst ? dst : out, add};
-  hipLaunchKernelGGL(k_spectral_back, dim3((unsigned)sp->h, BACK_GROUPS), dim3(256), 0,
-                     ctx->stream, b);
+  if (sp->w > MAX_SIDE)
+    hipLaunchKernelGGL(k_spectral_back_wide, dim3(8u * (unsigned)(sp->nbx * ((sp->h + 7) / 8))),
+                       dim3(64 * BACK_WIDE_WAVES), 0, ctx->stream, b);
+  else
+    hipLaunchKernelGGL(k_spectral_back, dim3((unsigned)sp->h, BACK_GROUPS), dim3(256), 0,
+                       ctx->stream, b);
   IEN_HIP(hipGetLastError());
   return IEN_OK;
 }
 
 size_t spectral_r_floats(const ien_spectral *sp) { return (size_t)sp->h * sp->w * SPEC; }
 size_t spectral_u_floats(const ien_spectral *sp) { return (size_t)sp->h * sp->half * SPEC2; }
+bool spectral_fits(size_t height, size_t width) {
+  return height >= 1 && width >= 1 && height <= LONG_SIDE && width <= LONG_SIDE;
+}
 
-}  // namespace ien
-
-extern "C" {
-
-ien_status ien_spectral_new(ien_ctx *ctx, size_t height, size_t width, ien_spectral **out) {
-  IEN_CHECK(ctx && out, IEN_ERR_INPUT, "null argument");
+ien_status spectral_new(ien_ctx *ctx, size_t height, size_t width, ien_spectral **out) {
   *out = nullptr;
-  IEN_CHECK(height >= 1 && width >= 1 && height <= MAX_SIDE && width <= MAX_SIDE, IEN_ERR_INPUT,
-            "spectral unit of %zu x %zu (sides 1 .. %d)", width, height, MAX_SIDE);
+  IEN_CHECK(spectral_fits(height, width), IEN_ERR_INPUT, "spectral unit of %zu x %zu (sides 1 .. %d)",
+            width, height, LONG_SIDE);
   IEN_HIP(hipSetDevice(ctx->device));
   const int h = (int)height, w = (int)width, half = w / 2 + 1;
   ien_spectral *sp = new ien_spectral;
@@ -742,7 +1177,9 @@ ien_status ien_spectral_new(ien_ctx *ctx, size_t height, size_t width, ien_spect
   sp->mb = (w + 31) / 32;
   sp->nba = (2 * h + 31) / 32;
   sp->nbx = (w + 31) / 32;
-  const double tau = 6.283185307179586476925, s = 1.0 / std::sqrt((double)h * w);
+  const double s = 1.0 / std::sqrt((double)h * w);
+  // (cos, sin) of 2 pi j / n once each: a table asks for n^2 of them.
+  const std::vector<double> trig_w = circle(w), trig_h = circle(h);
   const int xp = sp->xp, yp = sp->yp;
   // Row transform (A operand, rows m of R): cos for the real parts of
   // columns m < half, -sin for the imaginary parts of columns m - half + 1.
@@ -750,18 +1187,18 @@ ien_status ien_spectral_new(ien_ctx *ctx, size_t height, size_t width, ien_spect
     const int term = kk / xp, x = kk % xp;
     if (m >= w || x >= w) return 0;
     const int col = m < half ? m : m - half + 1;
-    const double a = tau * (double)((long)col * x % w) / w;
-    return split_half(m < half ? std::cos(a) : -std::sin(a), term);
+    const double *t = &trig_w[2 * (col * x % w)];
+    return split_half(m < half ? t[0] : -t[1], term);
   });
-  // Column transform (B operand, columns (part', ky)), x 1 / sqrt(h w) x 64:
+  // Column transform (B operand, columns (part', ky)), x 1 / sqrt(h w) over R's scale:
   // (a + i b) e^{-i theta}.  K: (term, part, y), terms hi, lo.
   const std::vector<uint16_t> ta = operand(sp->nba, 4 * yp / 16, [&](int n, int kk) -> uint16_t {
     const int term = kk / (2 * yp), part = (kk % (2 * yp)) / yp, y = kk % yp;
     if (n >= 2 * h || y >= h) return 0;
     const int pp = n / h, ky = n % h;
-    const double a = tau * (double)((long)ky * y % h) / h, c = std::cos(a), sn = std::sin(a);
+    const double c = trig_h[2 * (ky * y % h)], sn = trig_h[2 * (ky * y % h) + 1];
     const double v = pp == 0 ? (part == 0 ? c : sn) : (part == 0 ? -sn : c);
-    return split_half(v * s * 64.0, term);
+    return split_half(v * s / r_scale(w), term);
   });
   // Inverse columns (B operand, columns (part', y)): (a + i b) e^{+i theta}.
   // K: (term, part, ky), terms hi, lo.
@@ -769,7 +1206,7 @@ ien_status ien_spectral_new(ien_ctx *ctx, size_t height, size_t width, ien_spect
     const int term = kk / (2 * yp), part = (kk % (2 * yp)) / yp, ky = kk % yp;
     if (n >= 2 * h || ky >= h) return 0;
     const int pp = n / h, y = n % h;
-    const double a = tau * (double)((long)ky * y % h) / h, c = std::cos(a), sn = std::sin(a);
+    const double c = trig_h[2 * (ky * y % h)], sn = trig_h[2 * (ky * y % h) + 1];
     const double v = pp == 0 ? (part == 0 ? c : -sn) : (part == 0 ? sn : c);
     return split_half(v, term);
   });
@@ -782,8 +1219,8 @@ ien_status ien_spectral_new(ien_ctx *ctx, size_t height, size_t width, ien_spect
     if (x >= w || m >= w) return 0;
     const int col = m < half ? m : m - half + 1;
     const double wk = (col == 0 || 2 * col == w) ? 1.0 : 2.0;
-    const double a = tau * (double)((long)col * x % w) / w;
-    const double v = m < half ? wk * std::cos(a) : -wk * std::sin(a);
+    const double *t = &trig_w[2 * (col * x % w)];
+    const double v = m < half ? wk * t[0] : -wk * t[1];
     return split_half(v * s * 256.0, term);
   });
   auto put = [](uint16_t **d, const std::vector<uint16_t> &v) {
@@ -800,6 +1237,18 @@ ien_status ien_spectral_new(ien_ctx *ctx, size_t height, size_t width, ien_spect
   }
   *out = sp;
   return IEN_OK;
+}
+
+}  // namespace ien
+
+extern "C" {
+
+ien_status ien_spectral_new(ien_ctx *ctx, size_t height, size_t width, ien_spectral **out) {
+  IEN_CHECK(ctx && out, IEN_ERR_INPUT, "null argument");
+  *out = nullptr;
+  IEN_CHECK(height >= 1 && width >= 1 && height <= MAX_SIDE && width <= MAX_SIDE, IEN_ERR_INPUT,
+            "spectral unit of %zu x %zu (sides 1 .. %d)", width, height, MAX_SIDE);
+  return spectral_new(ctx, height, width, out);
 }
 
 void ien_spectral_free(ien_spectral *sp) {

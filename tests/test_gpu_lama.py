@@ -35,6 +35,14 @@ def test_lama_matches_oracle(ctx, oracle, tensors, h, w):
     assert_spread(got, want, what=f"{h}x{w}")
 
 
+# Maps with a side of 65 .. 128 at an eighth (the spectral branch's wide rows,
+# tall columns and both): the first and the last such side, odd lines, lines
+# that end within a block of 16 or 32, beside the smallest other side.
+@pytest.mark.parametrize("h,w", [(16, 520), (17, 1024), (520, 16), (1024, 25), (776, 24), (30, 680), (560, 610)])
+def test_lama_long_maps_match_oracle(ctx, oracle, tensors, h, w):
+    test_lama_matches_oracle(ctx, oracle, tensors, h, w)
+
+
 def test_lama_graph_progress_and_cancel(ctx, tensors):
     import torch
     import ien
