@@ -560,64 +560,8 @@ __global__ __launch_bounds__(256) void conv_mfma(ConvArgs a) {
     }
   }
 
-  // ---- split-K counted in per tile: this split's sums go out (16 bytes a
-  // lane per accumulator quarter, in register order, at device scope so
-  // that a split on another XCD reads them from memory), then the tile's
-  // counter; the split that brings it to ksplit returns it to zero, adds
-  // the tile's sums in split order and carries on with the epilogue ----
-  if (a.ksplit > 1 && a.part) {
-    int *last = (int *)lds_raw;  // (written after the barrier below: every wave is past its products)
-    constexpr int G = MBW * NBW * 4;  // 16-byte groups a thread
-    constexpr int SC1 = 16;           // cache policy bits of a device-scope access
-    const int z = blockIdx.y;
-    const long first = (long)blockIdx.x * a.ksplit;  // the tile's first split block
-    const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
-        a.part, (short)0, (int)((long)gridDim.x * a.ksplit * G * 4096), 0x00020000);
-    auto at = [&](int s, int g) { return (int)((((first + s) * G + g) * 256 + tid) * 16); };
-#pragma unroll
-    for (int i = 0; i < MBW; i++)
-#pragma unroll
-      for (int j = 0; j < NBW; j++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const float4v v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
-                             acc[i][j][4 * q + 3]};
-          __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)&v, pr, at(z, (i * NBW + j) * 4 + q),
-                                                 0, SC1);
-        }
-    wait_vm<0>();  // this thread's sums are out
-    __syncthreads();
-    if (tid == 0) {
-      const int done =
-          __hip_atomic_fetch_add(a.tile_count + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      *last = done == a.ksplit - 1;
-      if (*last) __hip_atomic_store(a.tile_count + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    if (!*last) return;
-    // The sums in split order, this split's own read back too (the order,
-    // and so the result, must not depend on which split came last).
-#pragma unroll
-    for (int i = 0; i < MBW; i++)
-#pragma unroll
-      for (int j = 0; j < NBW; j++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-    for (int s = 0; s < a.ksplit; s++) {
-#pragma unroll
-      for (int i = 0; i < MBW; i++)
-#pragma unroll
-        for (int j = 0; j < NBW; j++)
-#pragma unroll
-          for (int q = 0; q < 4; q++) {
-            const u32x4 raw =
-                __builtin_amdgcn_raw_buffer_load_b128(pr, at(s, (i * NBW + j) * 4 + q), 0, SC1);
-            const float4v v = *(const float4v *)&raw;
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[i][j][4 * q + e] += v[e];
-          }
-    }
-  }
+  // (Every wave is past its products after count_in's first barrier.)
+  if (a.ksplit > 1 && a.part && !count_in<MBW, NBW, 256>(a, acc, (int *)lds_raw, tid)) return;
 
   // ---- epilogue -----------------------------------------------------------
   // Bias (and, when not accumulating, the activation) in the accumulators;
@@ -1270,6 +1214,25 @@ static ien_status run_cfg(ien_ctx *ctx, ConvArgs a) {
 // that divides the channel count.
 static int pick_ck(int c) { return c % 64 == 0 ? 64 : c % 32 == 0 ? 32 : 16; }
 
+// Microseconds that an NHWC 3 x 3 stride-1 product of 64s of channels takes
+// here, by the number of its 4 x 32 x 64 tiles: one round of double-buffered
+// workgroups (with their splits), two a CU on 16-channel chunks, or
+// single-buffered ones.  Fitted to sweeps on an idle MI355X (us, measured:
+// 64 x 96, 256 -> 256 14.5; 85 x 125, 512 -> 128 25.5; 128 x 192, 128 -> 128
+// 12.8; 95 x 95, 512 -> 256 34; 85 x 125, 128 -> 384 19.7; 71 x 472,
+// 512 -> 128 65; 200 x 200, 256 -> 256 70).
+static double general_us(const ien_ctx *ctx, const ConvArgs &a) {
+  const long tiles = (long)((a.OH + 3) / 4) * ((a.OW + 31) / 32) * ((a.N + 63) / 64);
+  const int chunks = a.C / 32;
+  const double round = (double)tiles / ctx->cus;
+  if (round <= 1) {
+    const int splits = round <= 0.25 ? (int)std::min<long>(chunks / 2, ctx->cus / tiles) : 1;
+    return splits > 1 ? 8.5 + 1.2 * ((chunks + splits - 1) / splits) : 5.5 + 1.2 * chunks;
+  }
+  if (round <= 2) return 5.4 + 1.85 * chunks;
+  return 4.6 + chunks * std::max(3.78, 1.5 * round);
+}
+
 ien_status launch_conv(ien_ctx *ctx, const ConvCall &c) {
   const ien_matrix *w = c.w;
   IEN_CHECK(w && w->d_packed, IEN_ERR_INPUT, "no weights");
@@ -1385,6 +1348,12 @@ ien_status launch_conv(ien_ctx *ctx, const ConvCall &c) {
     if (!vec) {
       if (nchw) return run_cfg<3, 1, 4, 32, 4, 2, 16, false, true>(ctx, a);
       return run_cfg<3, 1, 4, 32, 4, 2, 16, false, false>(ctx, a);
+    }
+    // 64s of channels: the pipelined kernel of a workgroup a CU, where it is
+    // estimated to be the faster one.
+    if (!nchw && ck == 64) {
+      const WidePlan plan = wide_plan(ctx, a);
+      if (plan.us > 0 && plan.us < general_us(ctx, a)) return launch_wide(ctx, a, plan);
     }
     // NHWC: 4 x 32 tiles and 32-channel chunks, so that the halo and weight
     // stages of three workgroups fit a CU's LDS and hide each other's load

@@ -240,6 +240,67 @@ __device__ __forceinline__ void dma16(const void *src, void *lds) {
   __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
 }
 
+// Split-K counted in per tile (a.part set): this split's sums go out (16 bytes
+// a lane per accumulator quarter, in register order, at device scope so that
+// a split on another XCD reads them from memory), then the tile's counter;
+// the split that brings it to ksplit returns it to zero, adds the tile's
+// sums in split order and gets true: it carries on with the epilogue.  `last`
+// is LDS that every wave is done with.
+template <int MB, int NB, int THREADS>
+__device__ __forceinline__ bool count_in(const ConvArgs &a, floatx16 (&acc)[MB][NB], int *last, int tid) {
+  constexpr int G = MB * NB * 4;  // 16-byte groups a thread
+  constexpr int SC1 = 16;         // cache policy bits of a device-scope access
+  const int z = blockIdx.y;
+  const long first = (long)blockIdx.x * a.ksplit;  // the tile's first split block
+  const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
+      a.part, (short)0, (int)((long)gridDim.x * a.ksplit * G * THREADS * 16), 0x00020000);
+  auto at = [&](int s, int g) { return (int)((((first + s) * G + g) * THREADS + tid) * 16); };
+#pragma unroll
+  for (int i = 0; i < MB; i++)
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const float4v v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
+                           acc[i][j][4 * q + 3]};
+        __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)&v, pr, at(z, (i * NB + j) * 4 + q), 0,
+                                               SC1);
+      }
+  wait_vm<0>();  // this thread's sums are out
+  __syncthreads();
+  if (tid == 0) {
+    const int done =
+        __hip_atomic_fetch_add(a.tile_count + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *last = done == a.ksplit - 1;
+    if (*last) __hip_atomic_store(a.tile_count + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!*last) return false;
+  // The sums in split order, this split's own read back too (the order, and
+  // so the result, must not depend on which split came last).
+#pragma unroll
+  for (int i = 0; i < MB; i++)
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+  for (int s = 0; s < a.ksplit; s++) {
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const u32x4 raw =
+              __builtin_amdgcn_raw_buffer_load_b128(pr, at(s, (i * NB + j) * 4 + q), 0, SC1);
+          const float4v v = *(const float4v *)&raw;
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[i][j][4 * q + e] += v[e];
+        }
+  }
+  return true;
+}
+
 // conv.hip: the pass after a split-K product -- the ksplit f32 partial sums
 // of `rows` x a.N outputs (rows `pitch` floats apart, split z after z rows
 // x pitch, in the context's workspace) added in order, then bias, old
@@ -266,6 +327,17 @@ bool narrow_supported(const ConvArgs &a, int ks, int stride, int nchw, int noff,
 ien_status launch_narrow(ien_ctx *ctx, ConvArgs a, int ks);
 bool few_supported(const ConvArgs &a, int ks, int stride, int nchw, int noff, int rows_mode);
 ien_status launch_few(ien_ctx *ctx, ConvArgs a, int ks);
+
+// conv_wide.hip: 3 x 3 stride-1 NHWC convolutions of 64s of channels with f16
+// outputs in 16-byte groups.
+// The estimated microseconds (of the best tile and split), or a
+// negative number where the kernel does not serve.
+struct WidePlan {
+  double us;
+  int tile, ksplit;
+};
+WidePlan wide_plan(const ien_ctx *ctx, const ConvArgs &a);
+ien_status launch_wide(ien_ctx *ctx, const ConvArgs &a, const WidePlan &plan);
 
 // conv_nchw.hip: 1x1 products of whole NCHW f16 planes into NCHW f16
 // planes (pixels a multiple of 8, 16-byte aligned planes), not accumulating.

@@ -123,6 +123,33 @@ def test_split_k_counted_in(ctx, oracle, act, acc):
     assert all(np.array_equal(r.view(np.uint32), runs[0].view(np.uint32)) for r in runs[1:])
 
 
+# The pipelined kernel of a workgroup a CU (channels in 64s; launch_conv takes
+# it where it is estimated to be faster): its 4 x 64, 4 x 128, 8 x 64 and
+# 8 x 128 tiles, with and without splits of the channels, on ragged maps, with
+# columns short of a 64 or 128, padded strides, old outputs, a range of rows
+# that starts and ends within a tile, and bit for bit the same when repeated.
+@pytest.mark.parametrize("h,w,c,n,pad,act,acc,row0,rows,sp", [
+    (85, 125, 512, 128, 1, 1, False, 0, None, 0),     # 4 x 64
+    (61, 67, 384, 136, 0, 0, True, 0, None, 8),       # 4 x 64, 8 columns in the last
+    (70, 77, 512, 128, 0, 1, True, 0, None, 8),       # 8 x 64, 4 splits
+    (95, 95, 512, 232, 0, 3, False, 0, None, 0),      # 4 x 128
+    (131, 163, 128, 200, 1, 2, True, 0, None, 16),    # 8 x 128, 56 of the last columns empty
+    (253, 250, 128, 64, 0, 1, False, 700, 62001, 0),  # 8 x 64, rows of part tiles
+    (2, 4000, 512, 128, 1, 0, False, 0, None, 0),     # two rows
+    (2500, 3, 192, 128, 0, 4, False, 0, None, 0),     # three columns
+])
+def test_conv3x3_wide(ctx, oracle, h, w, c, n, pad, act, acc, row0, rows, sp):
+    x, wt, b = case(h + w, h, w, c, n, 9)
+    rng = np.random.default_rng(h)
+    init = f16(rng.standard_normal((h * w, n)) * 0.5) if acc else None
+    slope = (0.1 + 0.2 * rng.random(n)).astype(np.float32)
+    want = want_cpu(oracle, x, wt, b, pad=pad, act=act, slope=slope, init=init)
+    got = [run_gpu(ctx, x, wt, b, pad=pad, act=act, slope=slope, init=init, row0=row0, rows=rows,
+                   stride_pad=sp) for _ in range(2)]
+    close(got[0], want[row0:None if rows is None else row0 + rows])
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+
+
 @pytest.mark.parametrize("c", [3, 4, 8, 16])
 def test_conv3x3_few_channels(ctx, oracle, c):
     x, wt, b = case(2, 11, 37, c, 64, 9)
