@@ -23,8 +23,18 @@
 //    per 16-byte item (8 channels of a row) the old output (loaded first,
 //    all at once) and the activation, one loop per activation: the order of
 //    gemm.rs:583-666.
-// Chunks of 32 channels keep the ring at 48 KiB (BN = 128), so several
+// Chunks of 32 channels keep the ring at 36 KiB (64 x 128 tiles), so several
 // workgroups share a CU and hide each other's latency.
+// Where the tiles leave no CU a second workgroup (KG = 2) nothing hides the
+// latency of four waves that wait for a chunk, read its fragments and
+// multiply them in turn (a 32-deep chunk took some 0.18 us, 0.05 of them
+// products).  There eight waves take a tile: chunks are 64 deep, each set of
+// four waves takes half of a chunk's steps, a chunk's fragments are read while
+// the one before is multiplied, and the two sets' sums meet in the epilogue's
+// LDS.  us, four waves (with their split-K) -> eight: 4096 x 1536 -> 384
+// 22.5 -> 11.6, 3269 x 1536 -> 384 19.5 -> 11.5, 1024 x 384 -> 384 7.8 -> 5.9,
+// 949 x 2048 -> 512 16.8 -> 13.0.  Over a CU's worth of tiles the four waves
+// stay the faster ones (24576 x 128 -> 512 16.7 against 20.5).
 // Tiles are dealt XCD-aware with N fastest, so a tile row's x stays in its
 // XCD's L2 for every column tile.
 // Planes: the rows may come from two maps (channels k1 .. K from x2, rows
@@ -68,7 +78,7 @@ struct RowsArgs {
   int pitch, kchunks;
 };
 
-template <int BM_, int BN, int KC>
+template <int BM_, int BN, int KC, int KG>
 struct RowsCfg {
   static constexpr int BM = BM_;
   static constexpr int SLOTS = KC / 8;                   // 16-byte slots per staged row
@@ -76,16 +86,20 @@ struct RowsCfg {
   static constexpr int B_BYTES = BN * KC * 2;
   static constexpr int STAGE = A_BYTES + B_BYTES;
   static constexpr int STAGES = 3;
-  static constexpr int A_LOADS = A_BYTES / 1024 / 4;     // per wave and chunk
-  static constexpr int B_LOADS = B_BYTES / 1024 / 4;
+  static constexpr int A_LOADS = A_BYTES / 1024 / (4 * KG);  // per wave and chunk
+  static constexpr int B_LOADS = B_BYTES / 1024 / (4 * KG);
   static constexpr int LPC = A_LOADS + B_LOADS;
   static constexpr int SP = BN + 4;                      // staged f32 row pitch
   static constexpr int LDS = STAGES * STAGE > 64 * SP * 4 ? STAGES * STAGE : 64 * SP * 4;
   static constexpr int WM = BN == 128 ? BM / 64 : 1;      // 32-row blocks per wave
   static constexpr int HALVES = BM / 64;                 // 64-row staging passes
-  static constexpr int ITEMS = BM * BN / 8 / 256;        // 16-byte output items per thread
-  static_assert(A_LOADS * 4 * 1024 == A_BYTES && B_LOADS * 4 * 1024 == B_BYTES, "load split");
+  static constexpr int THREADS = 256 * KG;
+  static constexpr int ITEMS = BM * BN / 8 / THREADS;    // 16-byte output items per thread
+  static_assert(A_LOADS * 4 * KG * 1024 == A_BYTES && B_LOADS * 4 * KG * 1024 == B_BYTES, "load split");
+  static_assert(KG == 1 || BM == 64, "two sets of waves share one staging pass");
 };
+
+constexpr int OOB = 0x7ffffff0;  // past every buffer
 
 // Slot of 16-byte chunk g of staged row r.
 template <int SLOTS>
@@ -98,13 +112,15 @@ __device__ __forceinline__ int swz(int r, int g) {
 // and is rounded again (a separate map addition after the product); 4: rows
 // are window tokens whose rounded result is added onto their map pixel
 // (ien_window_scatter_add after the product), tokens past the edge dropped.
-template <int BM, int BN, int KC, int MODE>
-__global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
-  using R = RowsCfg<BM, BN, KC>;
+template <int BM, int BN, int KC, int MODE, int KG>
+__global__ __launch_bounds__(256 * KG) void k_rows(RowsArgs a) {
+  using R = RowsCfg<BM, BN, KC, KG>;
+  constexpr int THREADS = R::THREADS;
   static_assert(BM == 128 || BN == 128, "64-row tiles are 128 columns wide");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[R::LDS];
   const int tid = threadIdx.x, lane = tid & 63, hf = lane >> 5, l32 = lane & 31;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wave8 & 3, kg = wave8 >> 2;  // kg: which part of each chunk's steps
   const int t = xcd_remap(blockIdx.x, gridDim.x);
   const int tm = t / a.tiles_n, tn = t - tm * a.tiles_n;
   const int m0 = tm * R::BM;
@@ -119,7 +135,7 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
   if constexpr (MODE == 1) {
 #pragma unroll
     for (int i = 0; i < R::A_LOADS; i++) {
-      const int m = m0 + (wave + 4 * i) * (1024 / (KC * 2)) + lane / R::SLOTS;
+      const int m = m0 + (wave8 + 4 * KG * i) * (1024 / (KC * 2)) + lane / R::SLOTS;
       const int yy = m / a.g2w;
       gpix[i] = 4 * yy * a.g2w + 2 * (m - yy * a.g2w);
     }
@@ -130,12 +146,13 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
   auto issue = [&](int lc, int s) {
     const int c = c_begin + lc;
     const unsigned base = l0 + s * R::STAGE;
+    const bool in = KG == 1 || lc < chunks;  // (past the end: zeros, so that every step issues as many loads)
     const bool second = c * KC >= a.k1;  // (uniform: k1 is a multiple of KC)
     const int4v sr = second ? xr2 : xr;
     const int rs = second ? a.xs2 : a.xs, c0 = second ? c * KC - a.k1 : c * KC;
 #pragma unroll
     for (int i = 0; i < R::A_LOADS; i++) {
-      const int d = wave + 4 * i;                 // KiB of the A stage
+      const int d = wave8 + 4 * KG * i;           // KiB of the A stage
       const int row = d * (1024 / (KC * 2)) + lane / R::SLOTS;
       const int slot = lane % R::SLOTS;
       const int g = swz<R::SLOTS>(row, slot);      // the chunk this slot holds
@@ -144,15 +161,15 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
         const int cin = a.K >> 2, q = c0 / cin;
         off = ((gpix[i] + (q >> 1) * 2 * a.g2w + (q & 1)) * rs + c0 - q * cin + 8 * g) * 2;
       }
-      dma_lds(sr, __builtin_amdgcn_readfirstlane(base + d * 1024), off);
+      dma_lds(sr, __builtin_amdgcn_readfirstlane(base + d * 1024), in ? off : OOB);
     }
 #pragma unroll
     for (int i = 0; i < R::B_LOADS; i++) {
-      const int f = wave + 4 * i;                 // fragment (j, q) of the chunk
+      const int f = wave8 + 4 * KG * i;           // fragment (j, q) of the chunk
       const int j = f / (KC / 16), q = f % (KC / 16);
       const int nb = tn * (BN / 32) + j, kb = c * (KC / 16) + q;
       dma_lds(wr, __builtin_amdgcn_readfirstlane(base + R::A_BYTES + f * 1024),
-               (nb * a.KB + kb) * 1024 + lane * 16);
+              in ? (nb * a.KB + kb) * 1024 + lane * 16 : OOB);
     }
   };
 
@@ -169,57 +186,128 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
 #pragma unroll
     for (int j = 0; j < 2; j++) acc[i][j] = floatx16{};
 
-  issue(0, 0);
-  if (chunks > 1) issue(1, 1);
-  for (int c = 0; c < chunks; c++) {  // c: this split's chunk index
-    if (c + 1 < chunks)
-      wait_vm<R::LPC>();  // all but chunk c + 1's loads
-    else
-      wait_vm<0>();
-    __syncthreads();  // chunk c visible; every wave is done with chunk c - 1
-    if (c + 2 < chunks) issue(c + 2, (c + 2) % 3);
-    const unsigned char *sa = lds + (c % 3) * R::STAGE;
-    const unsigned char *sb = sa + R::A_BYTES;
+  if constexpr (KG == 1) {
+    issue(0, 0);
+    if (chunks > 1) issue(1, 1);
+    for (int c = 0; c < chunks; c++) {  // c: this split's chunk index
+      if (c + 1 < chunks)
+        wait_vm<R::LPC>();  // all but chunk c + 1's loads
+      else
+        wait_vm<0>();
+      __syncthreads();  // chunk c visible; every wave is done with chunk c - 1
+      if (c + 2 < chunks) issue(c + 2, (c + 2) % 3);
+      const unsigned char *sa = lds + (c % 3) * R::STAGE;
+      const unsigned char *sb = sa + R::A_BYTES;
 #pragma unroll
-    for (int q = 0; q < KC / 16; q++) {
-      half8 af[R::WM], bf[2];
+      for (int q = 0; q < KC / 16; q++) {
+        half8 af[R::WM], bf[2];
 #pragma unroll
-      for (int i = 0; i < R::WM; i++) {
-        const int row = (wm * R::WM + i) * 32 + l32;
-        af[i] = *(const half8 *)(sa + row * KC * 2 + swz<R::SLOTS>(row, 2 * q + hf) * 16);
-      }
-#pragma unroll
-      for (int j = 0; j < 2; j++)
-        bf[j] = *(const half8 *)(sb + ((wn * 2 + j) * (KC / 16) + q) * 1024 + lane * 16);
-#pragma unroll
-      for (int i = 0; i < R::WM; i++)
+        for (int i = 0; i < R::WM; i++) {
+          const int row = (wm * R::WM + i) * 32 + l32;
+          af[i] = *(const half8 *)(sa + row * KC * 2 + swz<R::SLOTS>(row, 2 * q + hf) * 16);
+        }
 #pragma unroll
         for (int j = 0; j < 2; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
+          bf[j] = *(const half8 *)(sb + ((wn * 2 + j) * (KC / 16) + q) * 1024 + lane * 16);
+#pragma unroll
+        for (int i = 0; i < R::WM; i++)
+#pragma unroll
+          for (int j = 0; j < 2; j++)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
+      }
     }
+  } else {
+    // Fragments of chunk c: read while chunk c - 1 is multiplied.
+    constexpr int KS = KC / 16 / KG;  // this wave's 16-deep steps of a chunk
+    struct Frags {
+      half8 a[KS][R::WM], b[KS][2];
+    };
+    auto read = [&](Frags &f, int s) {
+      const unsigned char *sa = lds + s * R::STAGE;
+      const unsigned char *sb = sa + R::A_BYTES;
+#pragma unroll
+      for (int qq = 0; qq < KS; qq++) {
+        const int q = kg * KS + qq;
+#pragma unroll
+        for (int i = 0; i < R::WM; i++) {
+          const int row = (wm * R::WM + i) * 32 + l32;
+          f.a[qq][i] = *(const half8 *)(sa + row * KC * 2 + swz<R::SLOTS>(row, 2 * q + hf) * 16);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          f.b[qq][j] = *(const half8 *)(sb + ((wn * 2 + j) * (KC / 16) + q) * 1024 + lane * 16);
+      }
+    };
+    // Step c: chunk c + 1 has landed and every wave has chunk c's fragments in
+    // registers, so chunk c + STAGES takes its stage.
+    int stage = 0;
+    auto step = [&](int c, const Frags &now, Frags &next) {
+      wait_vm<(R::STAGES - 2) * R::LPC>();
+      lds_barrier();
+      issue(c + R::STAGES, stage);
+      stage = stage + 1 == R::STAGES ? 0 : stage + 1;
+      read(next, stage);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < KS; q++)
+#pragma unroll
+        for (int i = 0; i < R::WM; i++)
+#pragma unroll
+          for (int j = 0; j < 2; j++)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(now.a[q][i], now.b[q][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int s = 0; s < R::STAGES; s++) issue(s, s);
+    wait_vm<(R::STAGES - 1) * R::LPC>();
+    lds_barrier();
+    Frags f0, f1;
+    read(f0, 0);
+    for (int c = 0; c < chunks; c += 2) {  // (an odd count ends with a step of zeros)
+      step(c, f0, f1);
+      step(c + 1, f1, f0);
+    }
+    wait_vm<0>();
   }
   __syncthreads();  // every wave is done with the stages
 
+  // acc + bias as f32 rows in LDS, 64 rows at a time (the two sets of waves'
+  // sums one after the other), and a barrier.
+  float *st = (float *)lds;
+  const int owner = BM == 64 ? 0 : BN == 128 ? wm : wm >> 1;  // the 64 rows this wave computed
+  auto put = [&](int half, bool add, bool with_bias) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const float b = with_bias ? bias_r[j] : 0.0f;
+#pragma unroll
+      for (int i = 0; i < R::WM; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          float *s = st + ((wm * R::WM + i) * 32 - 64 * half + 8 * (r >> 2) + 4 * hf + (r & 3)) * R::SP +
+                     (wn * 2 + j) * 32 + l32;
+          *s = (add ? acc[i][j][r] + *s : acc[i][j][r]) + b;
+        }
+    }
+  };
+  auto stage_rows = [&](int half, bool with_bias) {
+    if constexpr (KG == 2) {
+      if (kg == 1) put(0, false, false);
+      __syncthreads();
+      if (kg == 0) put(0, true, with_bias);
+    } else if (owner == half) {
+      put(half, false, with_bias);
+    }
+    __syncthreads();
+  };
+
   if (a.part) {  // split-K: raw sums, 32 bytes per item
-    float *st = (float *)lds;
-    const int owner = BM == 64 ? 0 : BN == 128 ? wm : wm >> 1;
 #pragma unroll
     for (int half = 0; half < R::HALVES; half++) {
       if (half) __syncthreads();
-      if (owner == half) {
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-          for (int i = 0; i < R::WM; i++)
-#pragma unroll
-            for (int r = 0; r < 16; r++)
-              st[((wm * R::WM + i) * 32 - 64 * half + 8 * (r >> 2) + 4 * hf + (r & 3)) * R::SP +
-                 (wn * 2 + j) * 32 + l32] = acc[i][j][r];
-      }
-      __syncthreads();
+      stage_rows(half, false);
 #pragma unroll
       for (int e = half * R::ITEMS / R::HALVES; e < (half + 1) * R::ITEMS / R::HALVES; e++) {
-        const int v = tid + 256 * e, row = v / (BN / 8), c8 = 8 * (v % (BN / 8));
+        const int v = tid + THREADS * e, row = v / (BN / 8), c8 = 8 * (v % (BN / 8));
         if (m0 + row >= a.M) continue;
         const float *sr = st + (row - 64 * half) * R::SP + c8;
         float *q = a.part + ((long)blockIdx.y * a.M + m0 + row) * a.pitch + tn * BN + c8;
@@ -252,7 +340,7 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
   if constexpr (MODE == 4) {
 #pragma unroll
     for (int e = 0; e < R::ITEMS; e++) {
-      const int v = tid + 256 * e, row = v / (BN / 8), col = tn * BN + 8 * (v % (BN / 8));
+      const int v = tid + THREADS * e, row = v / (BN / 8), col = tn * BN + 8 * (v % (BN / 8));
       const uint16_t *q = m0 + row < a.M && col < a.N ? win_dst(m0 + row, col) : nullptr;
       old2[e] = *(const u32x4 *)(q ? q : a.y);
     }
@@ -260,7 +348,7 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
   if constexpr (MODE == 3) {
 #pragma unroll
     for (int e = 0; e < R::ITEMS; e++) {
-      const int v = tid + 256 * e, row = v / (BN / 8), col = tn * BN + 8 * (v % (BN / 8));
+      const int v = tid + THREADS * e, row = v / (BN / 8), col = tn * BN + 8 * (v % (BN / 8));
       const bool ok = m0 + row < a.M && col < a.N;
       old2[e] = *(const u32x4 *)(a.add2 + (ok ? (long)(m0 + row) * a.ys + col : 0));
     }
@@ -268,16 +356,15 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
   if (a.accumulate) {
 #pragma unroll
     for (int e = 0; e < R::ITEMS; e++) {
-      const int v = tid + 256 * e, row = v / (BN / 8), col = tn * BN + 8 * (v % (BN / 8));
+      const int v = tid + THREADS * e, row = v / (BN / 8), col = tn * BN + 8 * (v % (BN / 8));
       const bool ok = m0 + row < a.M && col < a.N;
       old[e] = *(const u32x4 *)(ok ? out_at(m0 + row, col) : a.y);
     }
   }
-  float *st = (float *)lds;
   auto store = [&](auto actf, int half) {
 #pragma unroll
     for (int e = half * R::ITEMS / R::HALVES; e < (half + 1) * R::ITEMS / R::HALVES; e++) {
-      const int v = tid + 256 * e, row = v / (BN / 8), c8 = 8 * (v % (BN / 8));
+      const int v = tid + THREADS * e, row = v / (BN / 8), c8 = 8 * (v % (BN / 8));
       const int col = tn * BN + c8;
       if (m0 + row >= a.M || col >= a.N) continue;
       uint16_t *dst = nullptr;
@@ -310,25 +397,10 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
         if (a.ydup) __builtin_memcpy(a.ydup + (long)(m0 + row) * a.ys + col, o, 16);
     }
   };
-  // acc + bias as f32 rows in LDS, 64 rows at a time.
-  const int owner = BM == 64 ? 0 : BN == 128 ? wm : wm >> 1;  // the 64 rows this wave computed
 #pragma unroll
   for (int half = 0; half < R::HALVES; half++) {
     if (half) __syncthreads();  // the first half is read
-    if (owner == half) {
-#pragma unroll
-      for (int j = 0; j < 2; j++) {
-        const int col = (wn * 2 + j) * 32 + l32;
-        const float b = bias_r[j];
-#pragma unroll
-        for (int i = 0; i < R::WM; i++)
-#pragma unroll
-          for (int r = 0; r < 16; r++)
-            st[((wm * R::WM + i) * 32 - 64 * half + 8 * (r >> 2) + 4 * hf + (r & 3)) * R::SP + col] =
-                acc[i][j][r] + b;
-      }
-    }
-    __syncthreads();
+    stage_rows(half, true);
     switch (a.act) {
       case IEN_ACT_RELU: store([&](float v, int) { return act_c<IEN_ACT_RELU>(v, 0.0f); }, half); break;
       case IEN_ACT_GELU: store([&](float v, int) { return act_c<IEN_ACT_GELU>(v, 0.0f); }, half); break;
@@ -343,30 +415,47 @@ __global__ __launch_bounds__(256) void k_rows(RowsArgs a) {
   }
 }
 
-// Split-K when the tiles leave three quarters of the CUs idle, or any CU
-// idle with K at least 1536 deep: about two workgroups per CU, each split at
-// least 256 deep.  (Splitting products that already fill most CUs, such as
-// SCUNet's 1024-deep fc2 over 192 tiles, cost more in partial sums and the
-// finishing pass than it gained.)
+// Eight waves a tile where a CU gets at most one of them (see above), in
+// whole 64-deep chunks of one plane or pixel.
+template <int BM, int MODE>
+bool paired(const ien_ctx *ctx, const RowsArgs &a) {
+  return BM == 64 && a.tiles <= ctx->cus && a.K % 64 == 0 && a.k1 % 64 == 0 && (MODE != 1 || a.K % 256 == 0);
+}
+
+// Split-K when the tiles leave three quarters of the CUs idle: about two
+// workgroups per CU, each split at least 256 deep, where that is estimated
+// to be faster.  A split launch and its finishing pass take some 7.5 us and
+// 2.4 more a million partial sums (100 x 4096 -> 256 8.6 us; 256 x 3072 -> 768
+// 14.0, 512 x 2048 -> 512 12.9, 949 x 2048 -> 512 17); one launch of eight
+// waves a tile 4.2 and 0.27 a 64-deep chunk (21.0, 17.2, 12.6, 13.0).
 template <int BM, int BN, int KC, int MODE = 0>
 ien_status launch(ien_ctx *ctx, RowsArgs a, const ConvArgs &c) {
   a.tiles_n = (a.N + BN - 1) / BN;
   a.tiles = (a.M + BM - 1) / BM * a.tiles_n;
-  const int chunks = a.K / KC;
+  int chunks = a.K / KC;
   a.pitch = a.tiles_n * BN;
   int ksplit = 1;
   // (The finishing pass writes one map, row by row; gathered rows are
   // split like any others.)
   const bool planes = a.k1 < a.K || a.n1 < a.N || MODE >= 2;
-  if (!planes && chunks >= 16 && (4 * a.tiles <= ctx->cus || (a.K >= 1536 && a.tiles < ctx->cus))) {
+  if (!planes && chunks >= 16 && 4 * a.tiles <= ctx->cus) {
     ksplit = std::min(chunks / 8, (2 * ctx->cus + a.tiles - 1) / a.tiles);
     while (ksplit > 1 && (size_t)ksplit * a.M * a.pitch > ctx->splitk_floats) ksplit--;
   }
+  bool pair = paired<BM, MODE>(ctx, a);
+  if (pair && ksplit > 1) {
+    pair = 4.2 + 0.27 * (a.K / 64) < 7.5 + 2.4e-6 * ksplit * a.M * a.pitch;
+    if (pair) ksplit = 1;
+  }
+  if (pair) chunks = a.K / 64;
   a.kchunks = (chunks + ksplit - 1) / ksplit;
   ksplit = (chunks + a.kchunks - 1) / a.kchunks;
   a.part = ksplit > 1 ? ctx->splitk : nullptr;
-  hipLaunchKernelGGL((k_rows<BM, BN, KC, MODE>), dim3((unsigned)a.tiles, (unsigned)ksplit), dim3(256), 0,
-                     ctx->stream, a);
+  const dim3 grid((unsigned)a.tiles, (unsigned)ksplit);
+  if constexpr (BM == 64) {
+    if (pair) hipLaunchKernelGGL((k_rows<BM, BN, 64, MODE, 2>), grid, dim3(512), 0, ctx->stream, a);
+  }
+  if (!pair) hipLaunchKernelGGL((k_rows<BM, BN, KC, MODE, 1>), grid, dim3(256), 0, ctx->stream, a);
   IEN_HIP(hipGetLastError());
   if (ksplit == 1) return IEN_OK;
   const ien_status st = splitk_finish(ctx, ksplit, a.M, a.pitch, c);
@@ -379,15 +468,17 @@ ien_status launch(ien_ctx *ctx, RowsArgs a, const ConvArgs &c) {
 
 }  // namespace
 
-// Tiles of 128 rows when they number at least 128, else 64-row tiles when
-// those number at least 96, or at least 8 with K 512 deep (split-K); below
-// that the general kernel serves.
 static long tiles_of(long rows, int bm, int n) { return (rows + bm - 1) / bm * ((n + 127) / 128); }
 
+// Any number of tiles that eight waves each can take (64s of channels: 104 x
+// 384 -> 384 7.4 us on the general kernel, 5.8 here; 145 x 1024 -> 256 10.4
+// and 8.4; 900 x 128 -> 128 5.4 and 5.0); else 128-row tiles when they number
+// at least 128, 64-row tiles when those number at least 96, or at least 8
+// with K 512 deep (split-K); below that the general kernel serves.
 bool rows_supported(const ConvArgs &a, long rows) {
   const bool aligned = (((uintptr_t)a.x) & 15) == 0 && (((uintptr_t)a.y) & 15) == 0;
   const long t64 = tiles_of(rows, 64, a.N);
-  const bool enough = tiles_of(rows, 128, a.N) >= 128 || t64 >= 96 || (t64 >= 8 && a.C >= 512);
+  const bool enough = a.C % 64 == 0 || tiles_of(rows, 128, a.N) >= 128 || t64 >= 96 || (t64 >= 8 && a.C >= 512);
   return aligned && !a.out_f32 && !a.out_nchw && a.C % 32 == 0 && a.N % 8 == 0 && a.xs % 8 == 0 &&
          a.ys % 8 == 0 && (long)a.xs * (rows + 128) * 2 <= 0x7fff0000L &&
          (long)a.NB * a.KB * 1024 <= 0x7fff0000L && enough;
