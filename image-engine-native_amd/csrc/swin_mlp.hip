@@ -1,6 +1,7 @@
 // swin_mlp.hip -- the Swin block's MLP half in one pass over the token rows
 // (crates/scunet-native/src/swin.rs:236-275, crates/birefnet-native/src/
-// swin.rs Mlp): x += fc2(GELU(fc1(LayerNorm(x)))), for c = 32, 64 and 96.
+// swin.rs Mlp): x += fc2(GELU(fc1(LayerNorm(x)))), for c = 32, 64 and 96 (large
+// maps of 96 channels by the kernel of strips at the end).
 //
 // One workgroup of 4 waves per 64 token rows:
 //  - LayerNorm (mean, then the mean square deviation, eps 1e-5: math.rs:
@@ -134,13 +135,26 @@ __global__ __launch_bounds__(256) void k_swin_mlp(MlpArgs a) {
     const uint16_t *w1 = a.w1 + ((size_t)(ch * 4 + wave) * a.kb1) * 512 + lane * 8;
 #pragma unroll
     for (int s = 0; s < S::KS1; s++) w1f[s] = *(const half8 *)(w1 + s * 512);
-    floatx16 h0 = {}, h1 = {};
+    // The units are the product's rows (the weights its A operand), so that a
+    // lane holds four consecutive units of one token: 8-byte writes, and the
+    // bias is where the sums start (us a block, with one product less in
+    // gelu_f: 96 channels at 256 x 256 104.7 -> 102, 64 at 256 x 384 57.3 -> 56.4).
+    floatx16 h0, h1;
+    const float *b1 = a.b1 + ch * MLP_CHUNK + wave * 32 + 4 * hf;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const float4 b = *(const float4 *)(b1 + 8 * q);
+      h0[4 * q] = h1[4 * q] = b.x;
+      h0[4 * q + 1] = h1[4 * q + 1] = b.y;
+      h0[4 * q + 2] = h1[4 * q + 2] = b.z;
+      h0[4 * q + 3] = h1[4 * q + 3] = b.w;
+    }
 #pragma unroll
     for (int s = 0; s < S::KS1; s++) {
       const half8 x0 = *(const half8 *)(xa + l32 * S::XP + 16 * s + 8 * hf);
       const half8 x1 = *(const half8 *)(xa + (32 + l32) * S::XP + 16 * s + 8 * hf);
-      h0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(x0, w1f[s], h0, 0, 0, 0);
-      h1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(x1, w1f[s], h1, 0, 0, 0);
+      h0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(w1f[s], x0, h0, 0, 0, 0);
+      h1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(w1f[s], x1, h1, 0, 0, 0);
     }
     // fc2's fragments for this chunk, in flight during the GELU.
     half8 w2f[S::TW][S::KS2];
@@ -152,14 +166,18 @@ __global__ __launch_bounds__(256) void k_swin_mlp(MlpArgs a) {
 #pragma unroll
       for (int s = 0; s < S::KS2; s++) w2f[j][s] = *(const half8 *)(w2 + s * 512);
     }
-    const int unit = ch * MLP_CHUNK + wave * 32 + l32;
-    const float bias1 = a.b1[unit];
     uint16_t *hbuf = hb + (ch & 1) * MLP_ROWS * S::HP;
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int row = 8 * (r >> 2) + 4 * hf + (r & 3);
-      hbuf[row * S::HP + wave * 32 + l32] = f2h(gelu_f(h0[r] + bias1));
-      hbuf[(32 + row) * S::HP + wave * 32 + l32] = f2h(gelu_f(h1[r] + bias1));
+    for (int q = 0; q < 4; q++) {
+      uint16_t o[8];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        o[j] = f2h(gelu_f(h0[4 * q + j]));
+        o[4 + j] = f2h(gelu_f(h1[4 * q + j]));
+      }
+      uint16_t *at = hbuf + l32 * S::HP + wave * 32 + 8 * q + 4 * hf;
+      __builtin_memcpy(at, o, 8);
+      __builtin_memcpy(at + 32 * S::HP, o + 4, 8);
     }
     __syncthreads();
     // fc2: rows 32 rb .. + 31 of the chunk against this wave's tiles.
@@ -211,8 +229,178 @@ __global__ __launch_bounds__(256) void k_swin_mlp(MlpArgs a) {
   }
 }
 
+// ---- the same a wave at a time ---------------------------------------------
+//
+// Each wave takes strips of 32 tokens through the whole MLP in registers, a
+// token a lane pair (lane l and l + 32 hold 8 of every 16 channels), with
+// nothing between the waves but the weights, which the workgroup holds in
+// LDS.  The weights are the products' A operands, so a product's result has
+// the token as its column, and what a lane holds of 32 hidden units (four of
+// every eight) is what it supplies to the next product: the reduction runs
+// over the units in that order, on both operands.  One lane swap at the end
+// brings the output to the order of the rows as they were loaded, so the
+// residual comes from registers.
+// Measured on a 256 x 256 map of 96 channels (windows of 12, us a block): 102
+// with the chunks above, whose 1024 workgroups each load the weights again and
+// wait at a barrier a chunk, 83 here.  What bounds it is VALU work: 22 issue
+// slots a GELU, 12.6 M values a CU's lanes at a time, some 14 us of it.
+template <int C>
+struct Strip {
+  static constexpr int KS1 = C / 16, UB = C / 8, CB = C / 32, KS2 = C / 4;
+  static constexpr int W1 = UB * KS1 * 1024, W2 = CB * KS2 * 1024;
+  static constexpr int VEC = W1 + W2;  // gamma, beta, b1, b2
+  static constexpr int LDS = VEC + 7 * C * 4;
+  static constexpr int WAVES = 8;  // one workgroup a CU: the weights of 96 channels take 144 KiB
+  static_assert(LDS <= 160 * 1024, "weights in LDS");
+};
+
+template <int C>
+__global__ __launch_bounds__(64 * Strip<C>::WAVES) void k_swin_mlp_strips(MlpArgs a) {
+  using S = Strip<C>;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[S::LDS];
+  float *vec = (float *)(lds + S::VEC);
+  const int tid = threadIdx.x, lane = tid & 63, hf = lane >> 5, l32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long strips = (a.rows + 31) / 32, step = (long)gridDim.x * S::WAVES, last = a.rows - 1;
+  long strip = (long)blockIdx.x * S::WAVES + wave;
+  u32x4 raw[S::KS1];
+  auto load = [&](long at) {
+    const uint16_t *row = a.map + min(at * 32 + l32, last) * a.stride + 8 * hf;
+#pragma unroll
+    for (int s = 0; s < S::KS1; s++) raw[s] = *(const u32x4 *)(row + 16 * s);
+  };
+  load(strip);
+  for (int f = wave; f < (S::W1 + S::W2) / 1024; f += S::WAVES) {
+    const bool second = f >= S::W1 / 1024;
+    dma16((second ? a.w2 + (long)(f - S::W1 / 1024) * 512 : a.w1 + (long)f * 512) + lane * 8, lds + f * 1024);
+  }
+  for (int i = tid; i < 7 * C; i += 64 * S::WAVES)
+    vec[i] = i < C ? a.gamma[i] : i < 2 * C ? a.beta[i - C] : i < 6 * C ? a.b1[i - 2 * C] : a.b2[i - 6 * C];
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the direct-to-LDS loads have landed
+  __syncthreads();
+  for (; strip < strips; strip += step) {
+    // LayerNorm: a token's channels lie in two lanes.
+    half8 x[S::KS1];
+    {
+      float v[S::KS1][8], sum = 0.0f, sq = 0.0f;
+#pragma unroll
+      for (int s = 0; s < S::KS1; s++) {
+        uint16_t h[8];
+        __builtin_memcpy(h, &raw[s], 16);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          v[s][e] = h2f(h[e]);
+          sum += v[s][e];
+        }
+      }
+      sum += __shfl_xor(sum, 32);
+      const float mean = sum / (float)C;
+#pragma unroll
+      for (int s = 0; s < S::KS1; s++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          v[s][e] -= mean;
+          sq += v[s][e] * v[s][e];
+        }
+      sq += __shfl_xor(sq, 32);
+      const float inv = 1.0f / sqrtf(sq / (float)C + 1e-5f);
+#pragma unroll
+      for (int s = 0; s < S::KS1; s++) {
+        const float *g = vec + 16 * s + 8 * hf;
+        __builtin_amdgcn_sched_barrier(0);  // (not every row of them in registers at once)
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[s][e] = (_Float16)(v[s][e] * inv * g[e] + g[C + e]);
+      }
+    }
+    // Sums that start at the biases of 32 rows (four of every eight).
+    auto start = [&](const float *b) {
+      floatx16 acc;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const float4v f = *(const float4v *)(b + 8 * q + 4 * hf);
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[4 * q + j] = f[j];
+      }
+      return acc;
+    };
+    floatx16 z[S::CB];
+#pragma unroll
+    for (int c = 0; c < S::CB; c++) z[c] = start(vec + 6 * C + 32 * c);
+#pragma unroll 1
+    for (int u = 0; u < S::UB; u++) {
+      floatx16 h = start(vec + 2 * C + 32 * u);
+      const unsigned char *w1 = lds + u * S::KS1 * 1024 + lane * 16;
+#pragma unroll
+      for (int s = 0; s < S::KS1; s++)
+        h = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const half8 *)(w1 + s * 1024), x[s], h, 0, 0, 0);
+      half8 g[2];
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        if (i == 8) __builtin_amdgcn_sched_barrier(0);
+        g[i >> 3][i & 7] = (_Float16)gelu_f(h[i]);
+      }
+      // Units 4 hf + i and 8 + 4 hf + i of each 16: half of either of the
+      // packed fragment's lanes l32 and 32 + l32.
+      const unsigned char *w2 = lds + S::W1 + 2 * u * 1024 + l32 * 16 + 8 * hf;
+#pragma unroll
+      for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int c = 0; c < S::CB; c++) {
+          half8 w;
+          __builtin_memcpy(&w, w2 + (c * S::KS2 + t) * 1024, 8);
+          __builtin_memcpy((char *)&w + 8, w2 + (c * S::KS2 + t) * 1024 + 512, 8);
+          z[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, g[t], z[c], 0, 0, 0);
+        }
+    }
+    // A lane's channels 8 q + 4 hf .. of an even and the next odd q, to
+    // channels 16 s + 8 hf .. + 7: the even one's upper lanes change places
+    // with the odd one's lower ones.
+    const long row = strip * 32 + l32;
+    uint16_t *out = a.map + row * a.stride + 8 * hf;
+    u32x4 done[S::KS1];
+#pragma unroll
+    for (int s = 0; s < S::KS1; s++) {
+      uint16_t h[8];
+      __builtin_memcpy(h, &raw[s], 16);
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(z[s >> 1][8 * (s & 1) + j]),
+                                                        __float_as_uint(z[s >> 1][8 * (s & 1) + 4 + j]), false, false);
+        v[j] = __uint_as_float(p[0]);
+        v[4 + j] = __uint_as_float(p[1]);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; e++) h[e] = f2h(v[e] + h2f(h[e]));
+      __builtin_memcpy(&done[s], h, 16);
+    }
+    if (strip + step < strips) load(strip + step);
+    if (row <= last) {
+#pragma unroll
+      for (int s = 0; s < S::KS1; s++) *(u32x4 *)(out + 16 * s) = done[s];
+    }
+  }
+}
+
+template <int C>
+ien_status launch_strips(ien_ctx *ctx, const MlpArgs &a) {
+  constexpr int W = Strip<C>::WAVES;
+  const long groups = ((a.rows + 31) / 32 + W - 1) / W;
+  hipLaunchKernelGGL(k_swin_mlp_strips<C>, dim3((unsigned)std::min<long>(groups, ctx->cus)), dim3(64 * W), 0,
+                     ctx->stream, a);
+  IEN_HIP(hipGetLastError());
+  return IEN_OK;
+}
+
 template <int C>
 ien_status launch(ien_ctx *ctx, const MlpArgs &a) {
+  // Strips from four a CU (40000 rows 80 -> 68 us a block, 32400 58.0 -> 57.5);
+  // below that a strip's own latency shows (15936 38 against 42).  Not 64
+  // channels: more small workgroups fit a CU above (65536 rows 39.7 against
+  // 43.7).
+  if constexpr (C == 96) {
+    if (a.rows >= 128L * ctx->cus) return launch_strips<C>(ctx, a);
+  }
   const long blocks = (a.rows + MLP_ROWS - 1) / MLP_ROWS;
   hipLaunchKernelGGL(k_swin_mlp<C>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, a);
   IEN_HIP(hipGetLastError());

@@ -103,3 +103,30 @@ def test_swin_block_relative_bias(ctx, oracle, c, window, shift, masked, size):
     err = np.abs(got - want)
     assert err.max() < 5e-2 and np.sqrt(np.mean(err ** 2)) < 6e-3, (err.max(), np.sqrt(np.mean(err ** 2)))
     blk.free()
+
+
+# Maps of 96 channels large enough for the MLP's kernel of 32-token strips
+# (from 128 rows a CU): a part strip at the end, and more strips than waves.
+# Against the oracle at 4 f16 ulps of the peak (2^-10 each), twice the small
+# maps' bound for the tail of a hundred times as many values.
+@pytest.mark.parametrize("h,w", [(182, 181), (257, 256)])
+def test_swin_mlp_strips(ctx, oracle, h, w):
+    import torch
+    import ien
+
+    rng = np.random.default_rng(h)
+    c, stride = 96, 104
+    wt = block_weights(rng, c, 7)
+    blk = ien.Swin(ctx, c, 7, 3, -100.0, wt)
+    x = rng.standard_normal((h, w, c)).astype(np.float16)
+    md = torch.full((h * w, stride), 3.0, dtype=torch.float16, device="cuda")
+    md[:, :c] = torch.from_numpy(x.reshape(h * w, c)).cuda()
+    blk.run(md, stride, h, w)
+    torch.cuda.synchronize()
+    got = md.float().cpu().numpy()
+    blk.free()
+    assert np.all(got[:, c:] == 3.0)
+    want = oracle_block(oracle, x.astype(np.float32), 7, 3, -100.0, wt)
+    err = np.abs(got[:, :c].reshape(h, w, c) - want)
+    assert err.max() < 4 * 2.0**-10 * max(1.0, float(np.abs(want).max())), err.max()
+    assert np.sqrt(np.mean(err ** 2)) < 1e-3
