@@ -75,10 +75,23 @@ struct WideCfg {
   }
 };
 
-template <int TR, int NW, int KG, int S>
-__global__ __launch_bounds__(512, 2) void conv_wide(ConvArgs a) {
+// A doubling transposed convolution (UP): its four output phases' products
+// over offset taps in one launch.  Phase p = 2 py + px reads the pixel and,
+// where py or px is set, the next one down or across: nine (phase, tap)
+// pairs in all, which take the nine taps' places above; the phases' sums stay
+// in registers side by side and the halo serves them all.
+struct UpWeights {
+  const uint16_t *wp[4];
+  const float *bias[4];
+  int kb[4];  // 16-deep blocks of each matrix
+};
+constexpr int UP_PHASE[9] = {0, 1, 1, 2, 2, 3, 3, 3, 3}, UP_TAP[9] = {0, 0, 1, 0, 1, 0, 1, 2, 3};
+constexpr int UP_DY[9] = {0, 0, 0, 0, 1, 0, 0, 1, 1}, UP_DX[9] = {0, 0, 1, 0, 0, 0, 1, 0, 1};
+
+template <int TR, int NW, int KG, int S, bool UP>
+__global__ __launch_bounds__(512, 2) void conv_wide(ConvArgs a, UpWeights up) {
   using Cfg = WideCfg<TR, NW, KG, S>;
-  constexpr int MB = Cfg::MB, MW = Cfg::MW;
+  constexpr int MB = Cfg::MB, MW = Cfg::MW, PH = UP ? 4 : 1, P = UP ? 0 : 1;  // phases, halo border
   __shared__ __attribute__((aligned(1024))) unsigned char lds[Cfg::LDS];
   const int bid = xcd_remap(blockIdx.x, gridDim.x);
   const int tpix = a.tiles_x * a.tiles_y;
@@ -92,7 +105,11 @@ __global__ __launch_bounds__(512, 2) void conv_wide(ConvArgs a) {
   constexpr int KS = 4 / KG;  // 16-deep steps of a tap for each wave
   const int nblk = tn * 2 * NW;  // first 32-channel block of the tile
   const int4v xr = uniform_rsrc(a.x, (long)a.H * a.W * a.xs * 2);
-  const int4v wr = uniform_rsrc(a.wp, (long)a.NB * a.KB * 1024);
+  int4v wr[PH];
+#pragma unroll
+  for (int q = 0; q < PH; q++)
+    wr[q] = UP ? uniform_rsrc(up.wp[q], (long)a.NB * up.kb[q] * 1024)
+               : uniform_rsrc(a.wp, (long)a.NB * a.KB * 1024);
   const unsigned l0 = lds_addr(lds);
   const int c_begin = (int)blockIdx.y * a.kchunks;
   const int chunks = min(a.C / 64 - c_begin, a.kchunks);
@@ -105,7 +122,7 @@ __global__ __launch_bounds__(512, 2) void conv_wide(ConvArgs a) {
   for (int i = 0; i < Cfg::PIECES; i++) {
     const int item = min(wave + 8 * i, Cfg::A_KIB - 1) * 64 + lane, p = item >> 3;
     const int hy = p / HC;
-    int iy = oy0 + hy - 1, ix = ox0 + p - hy * HC - 1;
+    int iy = oy0 + hy - P, ix = ox0 + p - hy * HC - P;
     bool ok = p < Cfg::HALO;
     if (iy < 0 || iy >= a.H || ix < 0 || ix >= a.W) {
       ok = ok && a.pad_reflect;
@@ -125,22 +142,23 @@ __global__ __launch_bounds__(512, 2) void conv_wide(ConvArgs a) {
   };
   // Weights of tap t of chunk c: fragments [32-channel block][16-deep step].
   auto issue_weights = [&](int c, int t, int slot) {
+    const int q = UP ? UP_PHASE[t] : 0, tap = UP ? UP_TAP[t] : t, kbs = UP ? up.kb[q] : a.KB;
 #pragma unroll
     for (int i = 0; i < NW; i++) {
       const int f = wave + 8 * i;
-      const int kb = t * (a.C / 16) + (c_begin + c) * 4 + (f & 3);
-      const int off = ((nblk + (f >> 2)) * a.KB + kb) * 1024 + lane * 16;
+      const int kb = tap * (a.C / 16) + (c_begin + c) * 4 + (f & 3);
+      const int off = ((nblk + (f >> 2)) * kbs + kb) * 1024 + lane * 16;
       const unsigned base = l0 + Cfg::B0 + (unsigned)slot * Cfg::SLOT + f * 1024;
-      dma_lds(wr, __builtin_amdgcn_readfirstlane(base), c < chunks ? off : OOB);
+      dma_lds(wr[q], __builtin_amdgcn_readfirstlane(base), c < chunks ? off : OOB);
     }
   };
 
-  floatx16 acc[MB][2] = {};
+  floatx16 acc[PH][MB][2] = {};
   // The fragments of step s (of this wave's) of tap (c, t): its rows and 64 channels.
   auto frag = [&](int c, int t, int slot, int s, half8 *av, half8 *bv) {
     const int ks = kg * KS + s;
     const unsigned char *ab = lds + (c & 1) * (Cfg::A_KIB * 1024);
-    const int dy = t / 3, dx = t - 3 * dy;
+    const int dy = UP ? UP_DY[t] : t / 3, dx = UP ? UP_DX[t] : t % 3;
 #pragma unroll
     for (int i = 0; i < MB; i++) {
       const int p = (mg * MB + i + dy) * HC + l32 + dx;
@@ -164,7 +182,7 @@ __global__ __launch_bounds__(512, 2) void conv_wide(ConvArgs a) {
   frag(0, 0, 0, 0, av[0], bv[0]);
   int slot = 0;
   auto tap = [&](int c, auto tc) {
-    constexpr int t = decltype(tc)::value;
+    constexpr int t = decltype(tc)::value, q = UP ? UP_PHASE[t] : 0;
     wait_vm<Cfg::pending(t)>();
     tap_barrier();  // the next tap (and at tap 8 the next halo) is in; every wave is done with the last one
     issue_weights(c + (t + S - 1) / 9, (t + S - 1) % 9, slot == 0 ? S - 1 : slot - 1);
@@ -182,7 +200,7 @@ __global__ __launch_bounds__(512, 2) void conv_wide(ConvArgs a) {
       for (int i = 0; i < MB; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[now][i], bv[now][j], acc[i][j], 0, 0, 0);
+          acc[q][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[now][i], bv[now][j], acc[q][i][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
     slot = next;
@@ -201,93 +219,106 @@ __global__ __launch_bounds__(512, 2) void conv_wide(ConvArgs a) {
   wait_vm<0>();  // (the loads past the end too: the stages reuse their LDS)
   __syncthreads();
 
-  if (KG == 1 && a.ksplit > 1 && !count_in<MB, 2, 512>(a, acc, (int *)lds, tid)) return;
+  if constexpr (KG == 1 && !UP)
+    if (a.ksplit > 1 && !count_in<MB, 2, 512>(a, acc[0], (int *)lds, tid)) return;
   __syncthreads();
 
   // Epilogue: acc + bias as f32 per wave in LDS, then 16-byte items of 8
   // channels of a pixel: old output, activation, f16, added map.
   float *stage = (float *)(lds + wave % (MW * NW) * Cfg::STAGE);
   constexpr int SP = Cfg::SP, ITEMS = MB * 4 / KG;
-  auto put = [&](bool add) {
+  auto put = [&](auto phase, bool add) {
+    constexpr int ph = decltype(phase)::value;
+    const float *bias = UP ? up.bias[ph] : a.bias;
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-      const float b = kg == 0 ? a.bias[(nblk + 2 * ng + j) * 32 + l32] : 0.0f;
+      const float b = kg == 0 ? bias[(nblk + 2 * ng + j) * 32 + l32] : 0.0f;
 #pragma unroll
       for (int i = 0; i < MB; i++)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           float *s = stage + (i * 32 + 8 * (r >> 2) + 4 * hi + (r & 3)) * SP + j * 32 + l32;
-          *s = (add ? acc[i][j][r] + *s : acc[i][j][r]) + b;
+          *s = (add ? acc[ph][i][j][r] + *s : acc[ph][i][j][r]) + b;
         }
     }
   };
-  if constexpr (KG == 1) {
-    put(false);
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes done
-    __builtin_amdgcn_wave_barrier();
-  } else {  // the second half of the steps, then the first half and the bias
-    if (kg == 1) put(false);
-    __syncthreads();
-    if (kg == 0) put(true);
-    __syncthreads();
-  }
   const int n0 = (nblk + 2 * ng) * 32 + 8 * (lane & 7);
-  int at[ITEMS];
-#pragma unroll
-  for (int t = 0; t < ITEMS; t++) {
-    const int q = (lane >> 3) + 8 * (KG * t + kg);
-    const int oy = oy0 + mg * MB + q / 32, ox = ox0 + (q & 31), p = oy * a.OW + ox;
-    const bool ok = oy < a.OH && ox < a.OW && p >= a.p_begin && p < a.p_end && n0 < a.N;
-    at[t] = ok ? (p - a.p_begin) * a.ys + n0 : -1;
-  }
   uint16_t *y = (uint16_t *)a.y;
-  u32x4 old[ITEMS], add[ITEMS];
-  if (a.accumulate) {
-#pragma unroll
-    for (int t = 0; t < ITEMS; t++) old[t] = *(const u32x4 *)(y + max(at[t], 0));
-  }
-  if (a.add2) {
-#pragma unroll
-    for (int t = 0; t < ITEMS; t++) add[t] = *(const u32x4 *)(a.add2 + max(at[t], 0));
-  }
-  auto store = [&](auto actf) {
+  auto finish = [&](auto phase) {
+    constexpr int ph = decltype(phase)::value;
+    if constexpr (KG == 1) {
+      put(phase, false);
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes done
+      __builtin_amdgcn_wave_barrier();
+    } else {  // the second half of the steps, then the first half and the bias
+      if (kg == 1) put(phase, false);
+      __syncthreads();
+      if (kg == 0) put(phase, true);
+      __syncthreads();
+    }
+    int at[ITEMS];
 #pragma unroll
     for (int t = 0; t < ITEMS; t++) {
-      if (at[t] < 0) continue;
-      const float *s = stage + ((lane >> 3) + 8 * (KG * t + kg)) * SP + 8 * (lane & 7);
-      const float4v s0 = *(const float4v *)s, s1 = *(const float4v *)(s + 4);
-      float v[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
-      uint16_t o[8], h[8];
-      if (a.accumulate) {
-        __builtin_memcpy(h, &old[t], 16);
+      const int q = (lane >> 3) + 8 * (KG * t + kg);
+      const int oy = oy0 + mg * MB + q / 32, ox = ox0 + (q & 31), p = oy * a.OW + ox;
+      const bool ok = oy < a.OH && ox < a.OW && p >= a.p_begin && p < a.p_end && n0 < a.N;
+      const int pixel = UP ? (2 * oy + (ph >> 1)) * 2 * a.OW + 2 * ox + (ph & 1) : p - a.p_begin;
+      at[t] = ok ? pixel * a.ys + n0 : -1;
+    }
+    u32x4 old[ITEMS], add[ITEMS];
+    if (a.accumulate) {
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[e] += h2f(h[e]);
+      for (int t = 0; t < ITEMS; t++) old[t] = *(const u32x4 *)(y + max(at[t], 0));
+    }
+    if (a.add2) {
+#pragma unroll
+      for (int t = 0; t < ITEMS; t++) add[t] = *(const u32x4 *)(a.add2 + max(at[t], 0));
+    }
+    auto store = [&](auto actf) {
+#pragma unroll
+      for (int t = 0; t < ITEMS; t++) {
+        if (at[t] < 0) continue;
+        const float *s = stage + ((lane >> 3) + 8 * (KG * t + kg)) * SP + 8 * (lane & 7);
+        const float4v s0 = *(const float4v *)s, s1 = *(const float4v *)(s + 4);
+        float v[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+        uint16_t o[8], h[8];
+        if (a.accumulate) {
+          __builtin_memcpy(h, &old[t], 16);
+#pragma unroll
+          for (int e = 0; e < 8; e++) v[e] += h2f(h[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] = f2h(actf(v[e], n0 + e));
+        if (a.add2) {
+          __builtin_memcpy(h, &add[t], 16);
+#pragma unroll
+          for (int e = 0; e < 8; e++) o[e] = f2h(h2f(o[e]) + h2f(h[e]));
+        }
+        __builtin_memcpy(y + at[t], o, 16);
       }
-#pragma unroll
-      for (int e = 0; e < 8; e++) o[e] = f2h(actf(v[e], n0 + e));
-      if (a.add2) {
-        __builtin_memcpy(h, &add[t], 16);
-#pragma unroll
-        for (int e = 0; e < 8; e++) o[e] = f2h(h2f(o[e]) + h2f(h[e]));
+    };
+    switch (a.act) {
+      case IEN_ACT_RELU: store([](float v, int) { return act_c<IEN_ACT_RELU>(v, 0.0f); }); break;
+      case IEN_ACT_GELU: store([](float v, int) { return act_c<IEN_ACT_GELU>(v, 0.0f); }); break;
+      case IEN_ACT_SIGMOID: store([](float v, int) { return act_c<IEN_ACT_SIGMOID>(v, 0.0f); }); break;
+      case IEN_ACT_PRELU: {
+        const float *sl = a.slope;
+        store([sl](float v, int n) { return v < 0.0f ? v * sl[n] : v; });
+        break;
       }
-      __builtin_memcpy(y + at[t], o, 16);
+      default: store([](float v, int) { return v; }); break;
     }
   };
-  switch (a.act) {
-    case IEN_ACT_RELU: store([](float v, int) { return act_c<IEN_ACT_RELU>(v, 0.0f); }); break;
-    case IEN_ACT_GELU: store([](float v, int) { return act_c<IEN_ACT_GELU>(v, 0.0f); }); break;
-    case IEN_ACT_SIGMOID: store([](float v, int) { return act_c<IEN_ACT_SIGMOID>(v, 0.0f); }); break;
-    case IEN_ACT_PRELU: {
-      const float *sl = a.slope;
-      store([sl](float v, int n) { return v < 0.0f ? v * sl[n] : v; });
-      break;
-    }
-    default: store([](float v, int) { return v; }); break;
+  finish(Const<0>{});
+  if constexpr (UP) {  // (a wave's stage is its own: its reads are done when its next writes are)
+    finish(Const<1>{});
+    finish(Const<2>{});
+    finish(Const<3>{});
   }
 }
 
-template <int TR, int NW, int KG, int S>
-ien_status launch(ien_ctx *ctx, ConvArgs a, int ksplit) {
+template <int TR, int NW, int KG, int S, bool UP = false>
+ien_status launch(ien_ctx *ctx, ConvArgs a, int ksplit, const UpWeights &up = {}) {
   using Cfg = WideCfg<TR, NW, KG, S>;
   a.ty_begin = a.p_begin / a.OW / TR;
   a.tiles_y = (a.p_end - 1) / a.OW / TR + 1 - a.ty_begin;
@@ -309,8 +340,8 @@ ien_status launch(ien_ctx *ctx, ConvArgs a, int ksplit) {
             IEN_ERR_INPUT, "%ld tiles in %d splits past the workspace", blocks, a.ksplit);
   a.part = ctx->splitk;
   a.tile_count = (int *)(ctx->splitk + ctx->splitk_floats);
-  hipLaunchKernelGGL((conv_wide<TR, NW, KG, S>), dim3((unsigned)blocks, (unsigned)a.ksplit), dim3(512), 0,
-                     ctx->stream, a);
+  hipLaunchKernelGGL((conv_wide<TR, NW, KG, S, UP>), dim3((unsigned)blocks, (unsigned)a.ksplit), dim3(512), 0,
+                     ctx->stream, a, up);
   IEN_HIP(hipGetLastError());
   return IEN_OK;
 }
@@ -346,7 +377,7 @@ constexpr double SPLIT_US = 6.0;
 WidePlan wide_plan(const ien_ctx *ctx, const ConvArgs &a) {
   WidePlan best{-1.0, 0, 1};
   if (a.C % 64 || a.N % 8 || a.ys % 8 || (((uintptr_t)a.y | (uintptr_t)a.add2) & 15) || a.out_nchw ||
-      a.out_f32 || a.phase || ctx->compact || (long)a.H * a.W * a.xs * 2 > 0x7fff0000L ||
+      a.out_f32 || ctx->compact || (long)a.H * a.W * a.xs * 2 > 0x7fff0000L ||
       (long)a.NB * a.KB * 1024 > 0x7fff0000L)
     return best;
   const int chunks = a.C / 64;
@@ -371,6 +402,40 @@ ien_status launch_wide(ien_ctx *ctx, const ConvArgs &a, const WidePlan &plan) {
     case 2: return launch<8, 2, 1, 4>(ctx, a, plan.ksplit);
     default: return launch<4, 1, 2, 8>(ctx, a, 1);
   }
+}
+
+// LaMa's doublings (1000 x 680 images, us): 85 x 125, 512 -> 256 as four
+// launches of the general kernel 112, here 43; 170 x 250, 256 -> 128 112 and
+// 48; 340 x 500, 128 -> 64 110 and 57.
+ien_status conv_up(ien_ctx *ctx, const uint16_t *x, int h, int w, int c, ien_matrix *const *phases, uint16_t *y,
+                   int ys, ien_act act) {
+  const int n = (int)phases[0]->n;
+  UpWeights up{};
+  for (int p = 0; p < 4; p++) {
+    const int taps = (1 + p / 2) * (1 + p % 2);
+    IEN_CHECK(phases[p]->d_packed && phases[p]->k == (size_t)taps * c && (int)phases[p]->n == n &&
+                  (long)phases[p]->nb * phases[p]->kb * 1024 <= 0x7fff0000L,
+              IEN_ERR_INPUT, "phase %d of %zu x %zu for %d channels", p, phases[p]->k, phases[p]->n, c);
+    up.wp[p] = phases[p]->d_packed;
+    up.bias[p] = phases[p]->d_bias;
+    up.kb[p] = phases[p]->kb;
+  }
+  IEN_CHECK(c % 64 == 0 && n % 8 == 0 && ys % 8 == 0 && ys >= n && (((uintptr_t)x | (uintptr_t)y) & 15) == 0 &&
+                (long)h * w * c * 2 <= 0x7fff0000L && 4L * h * w * ys < (1L << 31),
+            IEN_ERR_INPUT, "doubling of a %d x %d map, %d -> %d channels", w, h, c, n);
+  ConvArgs a{};
+  a.x = x;
+  a.H = a.OH = h;
+  a.W = a.OW = w;
+  a.C = a.xs = c;
+  a.p_end = h * w;
+  a.NB = phases[0]->nb;
+  a.KB = phases[3]->kb;
+  a.N = n;
+  a.y = y;
+  a.ys = ys;
+  a.act = act;
+  return launch<8, 1, 1, 8, true>(ctx, a, 1, up);
 }
 
 }  // namespace ien

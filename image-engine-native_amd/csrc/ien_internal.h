@@ -179,14 +179,16 @@ struct ConvCall {
   // ys apart, 16-byte aligned) added to each f16 result after the
   // activation, rounded again (the product followed by ien_add; it may be y).
   const uint16_t *add2 = nullptr;
-  // Optional, the same outputs and 3x3 or offset-tap products over whole
-  // maps: 1 + 2 py + px writes output pixel (y, x) to pixel (2 y + py,
-  // 2 x + px) of y, a map 2 OH x 2 OW with pixels ys apart (a transposed
-  // convolution's phase scattered as it is stored); 0 for none.
-  int phase = 0;
 };
 
 ien_status launch_conv(ien_ctx *ctx, const ConvCall &c);
+
+// conv_wide.hip: the four phases of a doubling transposed 3 x 3 convolution
+// (phase 2 py + px reads pixel (y, x) and, where py or px is set, the next one
+// down or across, taps in row order) over an h x w map of c channels (64s,
+// pixels c apart), each result stored at its pixel of the 2h x 2w map y.
+ien_status conv_up(ien_ctx *ctx, const uint16_t *x, int h, int w, int c, ien_matrix *const *phases, uint16_t *y,
+                   int ys, ien_act act);
 
 // conv_pair.hip: two 3x3 64 -> 64 convolutions with bias and PReLU in one
 // launch (x -> w1 -> w2 -> y, the intermediate map never stored): NHWC f16

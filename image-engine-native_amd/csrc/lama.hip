@@ -17,10 +17,9 @@ namespace {
 constexpr int LOCAL = 128, GLOBAL = 384, CHANNELS = 512, SPECTRAL = 192, BLOCKS = 18;
 constexpr int MULTIPLE = 8;
 
-// network.rs:271 PHASE_TAPS: output phase p = 2 py + px reads input offsets
-// (dy, dx) over the taps of py times those of px.
+// network.rs:271 PHASE_TAPS: output phase p = 2 py + px reads the taps of py
+// times those of px.
 constexpr int PHASE_COUNT[2] = {1, 2};
-constexpr int PHASE_OFFSET[2][2] = {{0, 0}, {0, 1}};
 
 ien_status matrix(ien_ctx *ctx, const TensorSource &take, const std::string &name, size_t k,
                   size_t n, bool bias, ien_matrix **out) {
@@ -119,41 +118,12 @@ ien_status ffc_run(Lama *l, const LamaFfc &f, const uint16_t *x, uint16_t *out, 
   return st;
 }
 
-// network.rs:279-335 Up::run: the four phase products, each storing its
-// outputs straight to their pixels of the doubled map (phase p = 2 py + px
-// to pixel (2 y + py, 2 x + px)).
+// network.rs:279-335 Up::run: the four phase products in one launch, each
+// storing its outputs straight to their pixels of the doubled map (phase
+// p = 2 py + px to pixel (2 y + py, 2 x + px)).
 ien_status up_run(Lama *l, ien_matrix *const *phases, const uint16_t *x, int h, int w, int cin,
                   int cout, uint16_t *y) {
-  for (int p = 0; p < 4; p++) {
-    const int py = p / 2, px = p % 2;
-    ConvCall cc;
-    cc.x = x;
-    cc.H = h;
-    cc.W = w;
-    cc.C = cin;
-    cc.xs = cin;
-    cc.noff = 0;
-    for (int a = 0; a < PHASE_COUNT[py]; a++)
-      for (int b = 0; b < PHASE_COUNT[px]; b++) {
-        cc.offy[cc.noff] = PHASE_OFFSET[py][a];
-        cc.offx[cc.noff] = PHASE_OFFSET[px][b];
-        cc.noff++;
-      }
-    cc.ks = 0;
-    cc.stride = 1;
-    cc.OH = h;
-    cc.OW = w;
-    cc.row0 = 0;
-    cc.rows = (long)h * w;
-    cc.w = phases[p];
-    cc.y = y;
-    cc.ys = cout;
-    cc.phase = 1 + p;
-    cc.act = IEN_ACT_RELU;
-    ien_status st = launch_conv(l->ctx, cc);
-    if (st != IEN_OK) return st;
-  }
-  return IEN_OK;
+  return conv_up(l->ctx, x, h, w, cin, phases, y, cout, IEN_ACT_RELU);
 }
 
 void free_maps(Lama &l) {
