@@ -285,6 +285,15 @@ ien_status lama_reserve(Lama *l, size_t pw, size_t ph, bool *grew) {
 // reads: FFC k - 1 reads the other map (or, for the second FFC of a
 // block, x, whose global part it only reads in its rows and local launches,
 // both before the wait).
+struct Serial {  // every branch on the context's stream while it lives
+  ien_ctx *ctx;
+  bool was;
+  Serial(ien_ctx *c, bool on) : ctx(c), was(c->serial_branches) { ctx->serial_branches = was || on; }
+  ~Serial() { ctx->serial_branches = was; }
+  Serial(const Serial &) = delete;
+  Serial &operator=(const Serial &) = delete;
+};
+
 template <class Done>
 ien_status ffc_pipeline(Lama *l, int h, int w, Done &done) {
   ien_ctx *ctx = l->ctx;
@@ -303,6 +312,14 @@ ien_status ffc_pipeline(Lama *l, int h, int w, Done &done) {
     return conv(ctx, c.x, h, w, LOCAL, CHANNELS, 3, 1, c.f->cross, c.out + LOCAL, CHANNELS,
                 IEN_ACT_NONE, 0);
   };
+  // Launched one by one, small maps keep the host busier than the GPU: there
+  // the branches' events cost more than their overlap gives (2.46 against
+  // 2.21 ms at 256 x 256, 2.63 against 2.03 at 128 x 96; 2.58 against 2.66 at
+  // 512 x 512, and replayed graphs gain at every size: 1.64 against 1.81 at
+  // 256 x 256).
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  IEN_HIP(hipStreamIsCapturing(ctx->stream, &cap));
+  const Serial serial(ctx, cap == hipStreamCaptureStatusNone && (long)h * w <= 1024);
   const bool split = !ctx->serial_branches;
   hipStream_t branch2 = ctx->branch[1];
   // The first cross convolution: x's local part is final now.
