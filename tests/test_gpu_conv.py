@@ -300,6 +300,14 @@ def test_stride2(ctx, oracle, pad):
     close(run_gpu(ctx, x, wt, b, step=2, pad=pad), want_cpu(oracle, x, wt, b, step=2, pad=pad))
 
 
+# Stride 2 with more tiles than CUs: 16-channel chunks of 32s and 64s of
+# channels, one tile past 256 and ragged edges.
+@pytest.mark.parametrize("h,w,c,n,pad", [(130, 511, 64, 128, 1), (515, 130, 32, 200, 0), (257, 259, 96, 130, 0)])
+def test_stride2_large_grid(ctx, oracle, h, w, c, n, pad):
+    x, wt, b = case(h, h, w, c, n, 9)
+    close(run_gpu(ctx, x, wt, b, step=2, pad=pad, act=1), want_cpu(oracle, x, wt, b, step=2, pad=pad, act=1))
+
+
 def test_reflect_3x3(ctx, oracle):
     x, wt, b = case(8, 9, 70, 64, 64, 9)
     close(run_gpu(ctx, x, wt, b, pad=1), want_cpu(oracle, x, wt, b, pad=1))
