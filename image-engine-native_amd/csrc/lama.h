@@ -54,8 +54,8 @@ ien_status spectral_front(const ien_spectral *sp, const uint16_t *x, long xs,
                           const ien_matrix *m_in, const ien_matrix *m_f, uint16_t *spectral,
                           float *r, float *u);
 // The front's two launches one at a time: the rows (spectral map and R),
-// then the columns (U; `z` holds the spectrum of a map over 64 rows, half x
-// (h rounded up to 32) pixels of 384 halves, and is not used otherwise).
+// then the columns (U; `z` holds the spectrum of a map with a side over 64,
+// half x (h rounded up to 32) pixels of 384 halves, and is not used otherwise).
 ien_status spectral_rows(const ien_spectral *sp, const uint16_t *x, long xs,
                          const ien_matrix *m_in, uint16_t *spectral, float *r);
 ien_status spectral_columns(const ien_spectral *sp, const ien_matrix *m_f, const float *r,

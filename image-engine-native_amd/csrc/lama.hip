@@ -241,8 +241,8 @@ ien_status lama_reserve(Lama *l, size_t pw, size_t ph, bool *grew) {
   free_maps(*l);
   *grew = true;
   // A spectrum has h8 (w8 / 2 + 1) <= h8 w8 = P / 64 pixels (w8 >= 2).
-  // The tall fused branch's spectrum (in filtered) has rows padded to blocks
-  // of 32: (w8 / 2 + 1)(h8 + 31) pixels at most, which is under S + 2200 for
+  // The fused branch's spectrum of a side over 64 (in filtered) has rows
+  // padded to blocks of 32: (w8 / 2 + 1)(h8 + 31) pixels at most, which is under S + 2200 for
   // sides up to 128 (h8 w8 / 2 + h8 + 15.5 w8 + 31).
   const size_t S = P / 64;
   auto alloc = [](uint16_t **p, size_t halves) { return hipMalloc((void **)p, halves * 2); };

@@ -8,11 +8,10 @@
 //   out       = ReLU(out + spectral spectral_out)            1x1, 192 -> 384, accumulated
 //
 // for maps of at most 64 x 64 (LaMa's eighth scale up to 512 x 512 images),
-// and in three or four for sides of up to 128 (the wide and tall kernels
-// below: a side over 64 takes its own variant of the launches that hold a
-// whole line of that direction).  The unfused path (fourier.hip and four
-// products) takes seven dependent launches, each a load -> compute -> store
-// chain of a few microseconds on a map of 1.5 MB; here:
+// and in four where a side is 65 .. 128 (the wide and tall kernels below).
+// The unfused path (fourier.hip and four products) takes seven dependent
+// launches, each a load -> compute -> store chain of a few microseconds on a
+// map of 1.5 MB; here:
 //
 //   front  (one workgroup per map row and 64-channel group): the spectral_in
 //          product for the row's pixels, bias, ReLU, f16 (the spectral map,
@@ -33,16 +32,19 @@
 //          and rounded to f16, then the spectral_out product accumulated onto
 //          the cross output with ReLU.
 //
-// Every product runs on v_mfma_f32_32x32x16_f16.  The transforms are real
-// matrix products with tables built in double on the host; to keep their
-// sums at f32 accuracy, an f32 operand v enters as the two halves
-// hi = f16(v), lo = f16(v - hi) and each table entry likewise, and a product
-// sums hi.hi + lo.hi + hi.lo (|error| about 2^-22 of the terms): the split is
-// one more stretch of the reduction (K) dimension.  f32 intermediates are
-// scaled by powers of two before the split (R by 2^-6, or 2^-7 for rows over
-// 64, U by 2^-8, undone in the tables) so that no half overflows.  The rounding points are those of
-// the unfused path: the spectral map, the spectrum and the filtered spectrum
-// in f16, the transforms' sums in f32.
+// Every product of channels runs on v_mfma_f32_32x32x16_f16.  The transforms
+// are real matrix products with tables built in double on the host, on the
+// same matrix cores with their operands split:
+//  - sides up to 64: an f32 operand v enters as the two halves hi = f16(v),
+//    lo = f16(v - hi) and each table entry likewise, and a product sums
+//    hi.hi + lo.hi + hi.lo: the split is one more stretch of the reduction
+//    (K) dimension.  f32 intermediates are scaled by powers of two before the
+//    split (R by 2^-6, U by 2^-8, undone in the tables) so that no half
+//    overflows; lo of a scaled value under 1 is an f16 subnormal, so an
+//    operand is off by up to 2^-25 of what its scale makes 1;
+//  - a side over 64: below, at those kernels.
+// The rounding points are those of the unfused path: the spectral map, the
+// spectrum and the filtered spectrum in f16, the transforms' sums in f32.
 //
 // The MFMA reduction dimension has to run along a lane's registers, so
 // every intermediate is laid out with the next reduction's index
@@ -53,6 +55,7 @@
 // ([n][ky]) for the inverse columns.
 
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "conv_common.h"
@@ -65,9 +68,7 @@ constexpr int SPEC = 192;      // spectral channels
 constexpr int SPEC2 = 384;     // spectrum values per pixel: re x 192 | im x 192
 constexpr int MAX_SIDE = 64;   // of the public plans, and of the kernels without a wide or tall variant
 constexpr int LONG_SIDE = 128;  // of the wide and tall kernels
-constexpr float USCALE = 1.0f / 256;
-// R's scale before the split: a row sums up to w f16 values.
-constexpr float r_scale(int w) { return w <= MAX_SIDE ? 1.0f / 64 : 1.0f / 128; }
+constexpr float RSCALE = 1.0f / 64, USCALE = 1.0f / 256;
 constexpr int COLUMN_GROUPS = 6;  // 32 channels a columns workgroup
 constexpr int BACK_GROUPS = 3;    // 128 output channels a back workgroup
 
@@ -100,7 +101,7 @@ struct FrontArgs {
   const uint16_t *w_in;
   int kb_in;
   const float *b_in;
-  const uint16_t *tf;  // A fragments [mb][2 xp / 16]: hi, then lo table
+  const uint16_t *tf;  // A fragments [mb][2 xp / 16]: hi, then lo table (x 2^11 for the wide kernel)
   uint16_t *s;         // spectral map, channel-major per row: [h][192][w]
   float *r;            // [h][w][192]
 };
@@ -212,7 +213,6 @@ struct ColumnArgs {
   int kb_f;
   const float *b_f;
   float *u;  // [h][half][384]
-  float rscale;
 };
 
 constexpr int RP = MAX_SIDE + 8;                        // halves per transposed R row
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(512) void k_spectral_columns(ColumnArgs p) {
         for (int cc = 0; cc < 4; cc++) {
           float f[8];
 #pragma unroll
-          for (int j = 0; j < 8; j++) f[j] = v[b][j][cc] * p.rscale;
+          for (int j = 0; j < 8; j++) f[j] = v[b][j][cc] * RSCALE;
           half8 vh, vl;
           split8(f, vh, vl);
           const int row = part * SPEC + 4 * c4 + cc;
@@ -410,7 +410,9 @@ __global__ __launch_bounds__(512) void k_spectral_columns(ColumnArgs p) {
 struct BackArgs {
   const float *u;
   int h, w, half, mp, nbx;  // mp: w rounded up to 16; nbx: 32-blocks of w
-  const uint16_t *tr;       // B fragments [nbx][2 mp / 16]: (hi | lo, m)
+  // B fragments [nbx][2 mp / 16]: (hi | lo, m); for the wide kernel
+  // [nbx][mp / 16][bf16 piece, largest first].
+  const uint16_t *tr;
   const uint16_t *s;        // spectral map [h][192][w]
   const uint16_t *wo;
   int kb_o;
@@ -420,6 +422,7 @@ struct BackArgs {
   // it after the ReLU and rounding, rounded again (or null).
   uint16_t *dst;
   const uint16_t *add;
+  float scale;  // 1 / sqrt(h w), for the wide kernel
 };
 
 constexpr int UP = MAX_SIDE + 8;
@@ -627,12 +630,49 @@ __global__ __launch_bounds__(256) void k_spectral_back(BackArgs p) {
 // LaMa's maps of images over 512 pixels a side.  On 125 x 85 (1000 x 680
 // images) the unfused chain took 113 us of launches, 80 of them in four line
 // passes on f32 MFMA (1/16 of the f16 rate) with a table load per step;
-// these four take 15.5 (front), 14.5 and 14.9 (columns) and 20 us (back),
-// beside the convolutions' streams.  What bounds them is latency: each is
-// one load -> split -> product -> store chain a CU, at a round or less of
-// workgroups.
+// these four take 14 (front), 18 (columns, two) and 20 us (back), beside the
+// convolutions' streams.  What bounds them is latency: each is one load ->
+// split -> product -> store chain a CU, at a round or less of workgroups.
+//
+// The unfused chain's transforms are sums of f32 products, and these keep
+// that accuracy:
+//  - An f32 operand (R, U) is the sum of three bf16 values, exactly, and so is
+//    each entry of its table to 24 bits; a product sums the six products of
+//    pieces that reach 2^-24 of it, the largest apart from the rest.  bf16 has
+//    f32's exponents, so nothing is scaled and no magnitude loses bits.
+//  - An f16 operand (the spectral map, the filtered spectrum) is whole; its
+//    table's entries are hi + lo 2^-11, two halves of normal size (23 bits),
+//    the two sums apart.
+//  - 1 / sqrt(h w) multiplies the f32 sums, so that the tables hold 1 as 1.
+// Measured against 64 bits on the same operands (2-norm over the result's,
+// 125 x 85, 128 x 128 and 97 x 33 maps), f32 MFMA passes and here: rows 5.0 ..
+// 8.1 and 4.3 .. 6.3e-8, inverse columns 1.7 .. 2.1 and 1.2 .. 1.7e-7; columns
+// and inverse rows, stored in f16, a quarter of the passes' misrounded values.
+// (Two plain halves an operand, as for sides up to 64: 1.1 .. 1.3 times the
+// passes' error on rows and some 5 on columns and inverse rows, 1000 x 680
+// images in 3.73 ms against 3.80.)
 
-// front over rows of 65 .. 128 pixels: eight waves, one 32-channel x 32-pixel
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+constexpr float LO = 1.0f / 2048;  // of the second half of an f16 table entry
+
+__device__ __forceinline__ bf16x8 ldb8(const uint16_t *p) { return *(const bf16x8 *)p; }
+__device__ __forceinline__ floatx16 mfma16(bf16x8 a, bf16x8 b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+// Eight f32 values as three bf16 pieces, largest first.
+__device__ __forceinline__ void split8(const float *v, bf16x8 *piece) {
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    float rest = v[j];
+#pragma unroll
+    for (int t = 0; t < 3; t++) {
+      piece[t][j] = (__bf16)rest;
+      rest -= (float)piece[t][j];
+    }
+  }
+}
+
+// front over rows of up to 128 pixels: eight waves, one 32-channel x 32-pixel
 // block of the product each, then one 32 x 32 block of the row transform
 // each.  A workgroup holds its row (96 KiB) and its group's weights (48 KiB),
 // one a CU; the table fragments stay in registers and the transposed
@@ -655,8 +695,8 @@ __global__ __launch_bounds__(512) void k_spectral_front_wide(FrontArgs p) {
   row_part(blockIdx.x, SPEC / 64, y, g);
   if (y >= p.h) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 31, hi = lane >> 5;
-  constexpr int KS = GLOBAL_C / 16, TS = 2 * LONG_SIDE / 16;
-  const int ks_t = p.xp / 8;
+  constexpr int KS = GLOBAL_C / 16, XS = LONG_SIDE / 16;
+  const int xsteps = p.xp / 16;
   {
     const uint16_t *row = p.x + (long)y * p.w * p.xs;
     for (int f = wave; f * 64 < 48 * p.w; f += 8) {
@@ -673,11 +713,14 @@ __global__ __launch_bounds__(512) void k_spectral_front_wide(FrontArgs p) {
   float4v bias[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) bias[q] = *(const float4v *)(p.b_in + 64 * g + blk * 32 + 8 * q + 4 * hi);
-  half8 tf[TS];
+  half8 thi[XS], tlo[XS];
   {
-    const uint16_t *tb = p.tf + (long)min(line, p.mb - 1) * ks_t * 512 + lane * 8;
+    const uint16_t *tb = p.tf + (long)min(line, p.mb - 1) * 2 * xsteps * 512 + lane * 8;
 #pragma unroll
-    for (int i = 0; i < TS; i++) tf[i] = ld8(tb + min(i, ks_t - 1) * 512);
+    for (int i = 0; i < XS; i++) {
+      thi[i] = ld8(tb + min(i, xsteps - 1) * 512);
+      tlo[i] = ld8(tb + (xsteps + min(i, xsteps - 1)) * 512);
+    }
   }
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the direct-to-LDS loads have landed
   __syncthreads();
@@ -708,33 +751,47 @@ __global__ __launch_bounds__(512) void k_spectral_front_wide(FrontArgs p) {
   __syncthreads();
   if (line < p.mb) {
     const int c = blk * 32 + col;
-    floatx16 d = {};
+    floatx16 d = {}, dl = {};
 #pragma unroll
-    for (int i = 0; i < TS; i++)
-      if (i < ks_t) d = mfma16(tf[i], ld8(st + c * SPW + (16 * i + 8 * hi) % p.xp), d);
+    for (int i = 0; i < XS; i++) {
+      if (i < xsteps) {
+        const half8 b = ld8(st + c * SPW + 16 * i + 8 * hi);
+        d = mfma16(thi[i], b, d);
+        dl = mfma16(tlo[i], b, dl);
+      }
+    }
     float *out = p.r + (long)y * p.w * SPEC + 64 * g + c;
 #pragma unroll
     for (int r = 0; r < 16; r++) {
       const int m = line * 32 + 8 * (r >> 2) + 4 * hi + (r & 3);
-      if (m < p.w) out[(long)m * SPEC] = d[r];
+      if (m < p.w) out[(long)m * SPEC] = d[r] + dl[r] * LO;
     }
   }
 }
 
-// columns over 65 .. 128 rows, in two launches (a column of all channels
+// columns over up to 128 rows, in two launches (a column of all channels
 // would not fit a CU, and every group would transform it again): the column
 // transform of 32 channels a workgroup into the f16 spectrum, then the
 // fourier product of 32 real and 32 imaginary output channels and their
 // inverse columns.  The spectrum lies in the product's A fragments,
 // z[k][ky / 32][c' / 16], so that a wave reads it a KiB at a time.
-constexpr int TALL_STEPS = LONG_SIDE / 16;
+//
+// The transform folds its rows: cos is even about row 0 and sin odd, so with
+// E = R[y] + R[h - y] and O = R[y] - R[h - y] (y < F = (h + 1) / 2, E = R[0]
+// at y = 0)
+//   Re Z[ky] = sum cos E_re + sin O_im,   Im Z[ky] = sum cos E_im - sin O_re:
+// half the products, with one table [cos | sin] for both.  Row h / 2 of an
+// even h takes the place of O at y = 0 (of Re's or Im's own part), where the
+// table holds (-1)^ky.
+constexpr int TALL_STEPS = LONG_SIDE / 16, FOLD_STEPS = LONG_SIDE / 32;
 constexpr int ZK = SPEC2 / 16;  // 16-deep steps of the product
 
 struct TallArgs {
   const float *r;
-  int h, w, half, yp, nba, kyb;  // kyb: 32-blocks of h
-  float rscale;
-  const uint16_t *ta, *tc;  // as ColumnArgs
+  int h, w, half, yp, fsteps, nba, kyb;  // fsteps: 16-deep steps of F; kyb: 32-blocks of h
+  float scale;  // 1 / sqrt(h w)
+  const uint16_t *ta;  // B fragments [kyb][cos | sin][bf16 piece, smallest first][fsteps]
+  const uint16_t *tc;  // B fragments [nba][part][hi | lo][yp / 16]
   const uint16_t *wf;
   int kb_f;
   const float *b_f;
@@ -743,69 +800,78 @@ struct TallArgs {
 };
 
 __global__ __launch_bounds__(512, 4) void k_spectral_tall(TallArgs p) {
-  // A fragments of R, [hi | lo][part][y step], written once by the wave
-  // that loads the step's rows.
-  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * TALL_STEPS * 1024];
+  // A fragments of the folded rows, [piece][Re | Im][E | O][step], E written
+  // by the wave that loads the step's rows of that part, O by the other's.
+  constexpr int PIECE = 4 * FOLD_STEPS * 1024;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[3 * PIECE];
   int k, g;
   row_part(blockIdx.x, COLUMN_GROUPS, k, g);
   if (k >= p.half) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 31, hi = lane >> 5;
-  const int ysteps = p.yp / 16, ks2 = 2 * ysteps;
-  const uint16_t *tb = p.ta + (long)min(wave, p.nba - 1) * 2 * ks2 * 512 + lane * 8;
-  half8 thi[TALL_STEPS], tlo[TALL_STEPS];
+  const int h = p.h, part = wave & 1, blk = wave >> 1;  // part and step, then part and 32 ky
+  // The table's cos pieces; each makes room for the sin piece after its use.
+  const uint16_t *tb = p.ta + (long)min(blk, p.kyb - 1) * 6 * p.fsteps * 512 + lane * 8;
+  bf16x8 t[3][FOLD_STEPS];
 #pragma unroll
-  for (int ys = 0; ys < TALL_STEPS; ys++) {
-    thi[ys] = ld8(tb + min(ys, ysteps - 1) * 512);
-    tlo[ys] = ld8(tb + (ks2 + min(ys, ysteps - 1)) * 512);
-  }
-  if (wave < ysteps) {
-    const int mim = (k >= 1 && k <= p.w - p.half) ? p.half + k - 1 : -1;
-    float v[2][8];
+  for (int q = 0; q < 3; q++)
 #pragma unroll
-    for (int part = 0; part < 2; part++) {
-      const int m = part ? mim : k, y0 = 16 * wave + 8 * hi;
+    for (int s = 0; s < FOLD_STEPS; s++) t[q][s] = ldb8(tb + (q * p.fsteps + min(s, p.fsteps - 1)) * 512);
+  if (blk < p.fsteps) {
+    // Where R[y][m] is (m of either part; none: the imaginary parts of the
+    // first and, for an even w, last column).
+    const int mim = k >= 1 && k <= p.w - p.half ? p.half + k - 1 : -1;
+    const int m = part ? mim : k, other = part ? k : mim;
+    float v[8], mirror[8];
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const bool ok = m >= 0 && y0 + j < p.h;
-        v[part][j] = p.r[ok ? ((y0 + j) * p.w + m) * SPEC + 32 * g + col : 0];
-        if (!ok) v[part][j] = 0.0f;
-      }
+    for (int j = 0; j < 8; j++) {
+      const int y = 16 * blk + 8 * hi + j, ym = y == 0 ? h >> 1 : h - y, mm = y == 0 ? other : m;
+      const bool in = y < (h + 1) >> 1, ok = in && m >= 0;
+      const bool okm = in && mm >= 0 && (y > 0 || (h & 1) == 0);
+      v[j] = p.r[ok ? (y * p.w + m) * SPEC + 32 * g + col : 0];
+      mirror[j] = p.r[okm ? (ym * p.w + mm) * SPEC + 32 * g + col : 0];
+      if (!ok) v[j] = 0.0f;
+      if (!okm) mirror[j] = 0.0f;
     }
+    float even[8], odd[8];
 #pragma unroll
-    for (int part = 0; part < 2; part++) {
-#pragma unroll
-      for (int j = 0; j < 8; j++) v[part][j] *= p.rscale;
-      half8 vh, vl;
-      split8(v[part], vh, vl);
-      unsigned char *at = lds + (part * TALL_STEPS + wave) * 1024 + lane * 16;
-      *(half8 *)at = vh;
-      *(half8 *)(at + 2 * TALL_STEPS * 1024) = vl;
+    for (int j = 0; j < 8; j++) {
+      const bool first = j == 0 && 16 * blk + 8 * hi == 0;
+      even[j] = first ? v[j] : v[j] + mirror[j];
+      odd[j] = first ? mirror[j] : part ? v[j] - mirror[j] : mirror[j] - v[j];
     }
+    bf16x8 piece[3];
+    split8(even, piece);
+    unsigned char *at = lds + blk * 1024 + lane * 16;
+#pragma unroll
+    for (int n = 0; n < 3; n++) *(bf16x8 *)(at + n * PIECE + 2 * part * FOLD_STEPS * 1024) = piece[n];
+    split8(odd, piece);
+#pragma unroll
+    for (int n = 0; n < 3; n++) *(bf16x8 *)(at + n * PIECE + (3 - 2 * part) * FOLD_STEPS * 1024) = piece[n];
   }
   __syncthreads();
-  if (wave >= p.nba) return;
-  floatx16 acc = {};
+  if (blk >= p.kyb) return;
+  floatx16 acc = {}, small = {};
 #pragma unroll
-  for (int part = 0; part < 2; part++)
+  for (int q = 0; q < 6; q++) {
+    const int piece = 2 - q % 3;  // of the table
 #pragma unroll
-    for (int ys = 0; ys < TALL_STEPS; ys++) {
-      if (ys < ysteps) {
-        const unsigned char *at = lds + (part * TALL_STEPS + ys) * 1024 + lane * 16;
-        const half8 ah = *(const half8 *)at, al = *(const half8 *)(at + 2 * TALL_STEPS * 1024);
-        acc = mfma16(ah, thi[ys], acc);
-        acc = mfma16(al, thi[ys], acc);
-        acc = mfma16(ah, tlo[ys], acc);
-        if (part == 0) {  // the imaginary part's fragments, over the real part's
-          thi[ys] = ld8(tb + (ysteps + ys) * 512);
-          tlo[ys] = ld8(tb + (ks2 + ysteps + ys) * 512);
-        }
+    for (int s = 0; s < FOLD_STEPS; s++) {
+      if (s < p.fsteps) {
+        const unsigned char *at = lds + ((2 * part + q / 3) * FOLD_STEPS + s) * 1024 + lane * 16;
+        const bf16x8 tq = t[q % 3][s];
+#pragma unroll
+        for (int n = 2 - piece; n > 0; n--) small = mfma16(*(const bf16x8 *)(at + n * PIECE), tq, small);
+        floatx16 &first = piece == 0 ? acc : small;
+        first = mfma16(*(const bf16x8 *)at, tq, first);
+        if (q < 3) t[q][s] = ldb8(tb + ((q + 3) * p.fsteps + s) * 512);
       }
     }
-  const int n = wave * 32 + col;
-  if (n < 2 * p.h) {
-    const int pp = n >= p.h, ky = n - pp * p.h;
-    uint16_t *zb = p.z + ((long)(k * p.kyb + (ky >> 5)) * ZK + (pp * SPEC + 32 * g) / 16) * 512 +
-                   (ky & 31) * 8 + 4 * hi;
+  }
+  const int ky = blk * 32 + col;
+  if (ky < h) {
+    uint16_t *zb = p.z + ((long)(k * p.kyb + blk) * ZK + (part * SPEC + 32 * g) / 16) * 512 + col * 8 + 4 * hi;
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[i] = (acc[i] + small[i]) * p.scale;
 #pragma unroll
     for (int q = 0; q < 4; q++)
       st4h(zb + (q >> 1) * 512 + (q & 1) * 256, acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
@@ -825,7 +891,7 @@ __global__ __launch_bounds__(512, 4) void k_spectral_tall_back(TallArgs p) {
   row_part(blockIdx.x, COLUMN_GROUPS, k, g);
   if (k >= p.half) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 31, hi = lane >> 5;
-  const int h = p.h, ysteps = p.yp / 16, ks2 = 2 * ysteps;
+  const int h = p.h, ysteps = p.yp / 16;
   constexpr int CG = SPEC / COLUMN_GROUPS, BATCH = ZK / 2;
   const int pb = wave >> 1, part = wave & 1;  // the product's block of rows, and part
   for (int f = wave; f < 2 * ZK; f += 8) {
@@ -860,16 +926,16 @@ __global__ __launch_bounds__(512, 4) void k_spectral_tall_back(TallArgs p) {
       }
     }
   }
-  const uint16_t *tb = p.tc + (long)min(wave, p.nba - 1) * 2 * ks2 * 512 + lane * 8;
+  const uint16_t *tb = p.tc + (long)min(wave, p.nba - 1) * 4 * ysteps * 512 + lane * 8;
   half8 thi[TALL_STEPS], tlo[TALL_STEPS];
 #pragma unroll
   for (int ys = 0; ys < TALL_STEPS; ys++) {
     thi[ys] = ld8(tb + min(ys, ysteps - 1) * 512);
-    tlo[ys] = ld8(tb + (ks2 + min(ys, ysteps - 1)) * 512);
+    tlo[ys] = ld8(tb + (ysteps + min(ys, ysteps - 1)) * 512);
   }
   __syncthreads();
   if (wave < p.nba) {
-    floatx16 d = {};
+    floatx16 d = {}, dl = {};
 #pragma unroll
     for (int fp = 0; fp < 2; fp++)
 #pragma unroll
@@ -877,13 +943,15 @@ __global__ __launch_bounds__(512, 4) void k_spectral_tall_back(TallArgs p) {
         if (ys < ysteps) {
           const half8 a = ld8(pt + (fp * CG + col) * SPW + ys * 16 + 8 * hi);
           d = mfma16(a, thi[ys], d);
-          d = mfma16(a, tlo[ys], d);
+          dl = mfma16(a, tlo[ys], dl);
           if (fp == 0) {
-            thi[ys] = ld8(tb + (ysteps + ys) * 512);
-            tlo[ys] = ld8(tb + (ks2 + ysteps + ys) * 512);
+            thi[ys] = ld8(tb + (2 * ysteps + ys) * 512);
+            tlo[ys] = ld8(tb + (3 * ysteps + ys) * 512);
           }
         }
       }
+#pragma unroll
+    for (int i = 0; i < 16; i++) d[i] += dl[i] * LO;
     const int n = wave * 32 + col;
 #pragma unroll
     for (int q = 0; q < 4; q++)
@@ -899,7 +967,7 @@ __global__ __launch_bounds__(512, 4) void k_spectral_tall_back(TallArgs p) {
   }
 }
 
-// back over rows of 65 .. 128 pixels: a workgroup of six waves takes 32 of
+// back over rows of up to 128 pixels: a workgroup of six waves takes 32 of
 // a row's pixels.  Wave w's inverse rows are those of channels 32 w ..: their
 // U goes straight into A fragments (a lane's eight columns of one channel,
 // each read 32 consecutive channels a half wave); then two 32-channel blocks
@@ -925,18 +993,21 @@ __global__ __launch_bounds__(64 * BACK_WIDE_WAVES, 3) void k_spectral_back_wide(
     const int q = tid + 64 * BACK_WIDE_WAVES * i, x = min(q / 48, w - 1 - x0);
     old[i] = *(const u32x4 *)(p.out + orow + (long)x * p.ys + 8 * (q % 48));
   }
-  const uint16_t *tb = p.tr + (long)xb * 2 * msteps * 512 + lane * 8;
+  const uint16_t *tb = p.tr + (long)xb * 3 * msteps * 512 + lane * 8;
   const float *ub = p.u + (long)y * p.half * SPEC2 + 32 * wave;
-  floatx16 acc = {};
+  floatx16 acc = {}, small = {};
+  bf16x8 t[2][3];  // the table's fragments, two steps ahead
+  auto table = [&](int ms) {
 #pragma unroll
-  for (int m4 = 0; m4 < MS; m4 += 4) {  // four steps' loads together
+    for (int n = 0; n < 3; n++) t[ms & 1][n] = ldb8(tb + (3 * min(ms, msteps - 1) + n) * 512);
+  };
+  table(0);
+  table(1);
+#pragma unroll
+  for (int m4 = 0; m4 < MS; m4 += 4) {  // four steps' loads of U together
     float f[4][8];
-    half8 thi[4], tlo[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const int ms = min(m4 + i, msteps - 1);
-      thi[i] = ld8(tb + ms * 512);
-      tlo[i] = ld8(tb + (msteps + ms) * 512);
 #pragma unroll
       for (int j = 0; j < 8; j++) {
         const int m = 16 * (m4 + i) + 8 * hi + j;
@@ -948,17 +1019,30 @@ __global__ __launch_bounds__(64 * BACK_WIDE_WAVES, 3) void k_spectral_back_wide(
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      if (m4 + i < msteps) {
+      const int ms = m4 + i;
+      if (ms < msteps) {
+        const bf16x8 *b = t[ms & 1];
+        bf16x8 a[3];
+        split8(f[i], a);
+        small = mfma16(a[0], b[2], small);
+        small = mfma16(a[1], b[1], small);
+        small = mfma16(a[2], b[0], small);
+        small = mfma16(a[0], b[1], small);
+        small = mfma16(a[1], b[0], small);
+        acc = mfma16(a[0], b[0], acc);
+        if (ms + 2 < MS) table(ms + 2);
+      }
+    }
+    if (m4 == 0) {  // (their registers are the next steps')
 #pragma unroll
-        for (int j = 0; j < 8; j++) f[i][j] *= USCALE;
-        half8 ah, al;
-        split8(f[i], ah, al);
-        acc = mfma16(ah, thi[i], acc);
-        acc = mfma16(al, thi[i], acc);
-        acc = mfma16(ah, tlo[i], acc);
+      for (int i = 0; i < ITEMS; i++) {
+        const int q = tid + 64 * BACK_WIDE_WAVES * i;
+        *(u32x4 *)(ob + (q / 48) * OBW + 8 * (q % 48)) = old[i];
       }
     }
   }
+#pragma unroll
+  for (int i = 0; i < 16; i++) acc[i] = (acc[i] + small[i]) * p.scale;
   uint16_t sv[16];
   const uint16_t *sc = p.s + ((long)y * SPEC + 32 * wave) * w;
 #pragma unroll
@@ -975,11 +1059,6 @@ __global__ __launch_bounds__(64 * BACK_WIDE_WAVES, 3) void k_spectral_back_wide(
     st4h(s2 + col * S2P + 32 * wave + 8 * q + 4 * hi, acc[4 * q] + h2f(sv[4 * q]),
          acc[4 * q + 1] + h2f(sv[4 * q + 1]), acc[4 * q + 2] + h2f(sv[4 * q + 2]),
          acc[4 * q + 3] + h2f(sv[4 * q + 3]));
-#pragma unroll
-  for (int i = 0; i < ITEMS; i++) {
-    const int q = tid + 64 * BACK_WIDE_WAVES * i;
-    *(u32x4 *)(ob + (q / 48) * OBW + 8 * (q % 48)) = old[i];
-  }
   if (p.add) {
 #pragma unroll
     for (int i = 0; i < ITEMS; i++) {
@@ -1048,6 +1127,26 @@ uint16_t split_half(double v, int term) {
   return term == 0 ? hi : f32_to_half(f - half_bits_to_float(hi));
 }
 
+// The halves of v = hi + lo 2^-11: term 0 and 1, lo of normal size.
+uint16_t split_scaled(double v, int term) {
+  const uint16_t hi = f32_to_half((float)v);
+  return term == 0 ? hi : f32_to_half((float)((v - half_bits_to_float(hi)) / LO));
+}
+
+// The bf16 pieces of v, largest first: term 0, 1 and 2.
+uint16_t split_bf16(double v, int term) {
+  uint32_t bits = 0;
+  for (int t = 0;; t++) {
+    const float f = (float)v;
+    std::memcpy(&bits, &f, 4);
+    bits = (bits + 0x7fff + ((bits >> 16) & 1)) & 0xffff0000u;  // nearest, ties to even
+    if (t == term) return (uint16_t)(bits >> 16);
+    float piece;
+    std::memcpy(&piece, &bits, 4);
+    v -= piece;
+  }
+}
+
 // Fragments of an MFMA operand: fragment (blk, ks) holds value(32 blk + l %
 // 32, 16 ks + 8 (l / 32) + i) at lane l, element i (the layout of both the A
 // operand, rows x k, and the B operand, columns x k).
@@ -1084,6 +1183,10 @@ using namespace ien;
 struct ien_spectral {
   ien_ctx *ctx = nullptr;
   int h = 0, w = 0, half = 0, xp = 0, yp = 0, mb = 0, nba = 0, nbx = 0;
+  // A side over 64: every launch is the wide or tall kernel's, whose tables
+  // are split otherwise.
+  bool wide = false;
+  float scale = 1.0f;  // 1 / sqrt(h w)
   uint16_t *d_tf = nullptr, *d_ta = nullptr, *d_tc = nullptr, *d_tr = nullptr;
 };
 
@@ -1099,7 +1202,7 @@ ien_status spectral_rows(const ien_spectral *sp, const uint16_t *x, long xs,
   ien_ctx *ctx = sp->ctx;
   FrontArgs a{x, (int)xs, sp->h, sp->w, sp->xp, sp->mb, m_in->d_packed, m_in->kb, m_in->d_bias,
               sp->d_tf, spectral, r};
-  if (sp->w > MAX_SIDE)
+  if (sp->wide)
     hipLaunchKernelGGL(k_spectral_front_wide, dim3(8u * (SPEC / 64) * (unsigned)((sp->h + 7) / 8)),
                        dim3(512), 0, ctx->stream, a);
   else
@@ -1113,9 +1216,10 @@ ien_status spectral_columns(const ien_spectral *sp, const ien_matrix *m_f, const
                             uint16_t *z, float *u) {
   ien_ctx *ctx = sp->ctx;
   const unsigned column_blocks = 8u * COLUMN_GROUPS * (unsigned)((sp->half + 7) / 8);
-  if (sp->h > MAX_SIDE) {
-    IEN_CHECK(z && ((uintptr_t)z & 15) == 0, IEN_ERR_INPUT, "spectrum buffer of a tall map");
-    TallArgs t{r, sp->h, sp->w, sp->half, sp->yp, sp->nba, (sp->h + 31) / 32, r_scale(sp->w),
+  if (sp->wide) {
+    IEN_CHECK(z && ((uintptr_t)z & 15) == 0, IEN_ERR_INPUT, "spectrum buffer of a map with a side over %d",
+              MAX_SIDE);
+    TallArgs t{r, sp->h, sp->w, sp->half, sp->yp, (sp->h + 31) / 32, sp->nba, (sp->h + 31) / 32, sp->scale,
                sp->d_ta, sp->d_tc, m_f->d_packed, m_f->kb, m_f->d_bias, z, u};
     hipLaunchKernelGGL(k_spectral_tall, dim3(column_blocks), dim3(512), 0, ctx->stream, t);
     IEN_HIP(hipGetLastError());
@@ -1124,7 +1228,7 @@ ien_status spectral_columns(const ien_spectral *sp, const ien_matrix *m_f, const
     return IEN_OK;
   }
   ColumnArgs c{r, sp->h, sp->w, sp->half, sp->yp, sp->nba, sp->d_ta, sp->d_tc, m_f->d_packed,
-               m_f->kb, m_f->d_bias, u, r_scale(sp->w)};
+               m_f->kb, m_f->d_bias, u};
   hipLaunchKernelGGL(k_spectral_columns, dim3(column_blocks), dim3(512), 0, ctx->stream, c);
   IEN_HIP(hipGetLastError());
   return IEN_OK;
@@ -1144,8 +1248,8 @@ ien_status spectral_back(const ien_spectral *sp, const ien_matrix *m_out, const 
   IEN_CHECK((((uintptr_t)dst | (uintptr_t)add) & 15) == 0, IEN_ERR_INPUT,
             "spectral output and added map 16-byte aligned");
   BackArgs b{u, sp->h, sp->w, sp->half, sp->xp, sp->nbx, sp->d_tr, spectral, m_out->d_packed,
-             m_out->kb, out, (int)ys, dst ? dst : out, add};
-  if (sp->w > MAX_SIDE)
+             m_out->kb, out, (int)ys, dst ? dst : out, add, sp->scale};
+  if (sp->wide)
     hipLaunchKernelGGL(k_spectral_back_wide, dim3(8u * (unsigned)(sp->nbx * ((sp->h + 7) / 8))),
                        dim3(64 * BACK_WIDE_WAVES), 0, ctx->stream, b);
   else
@@ -1178,9 +1282,12 @@ ien_status spectral_new(ien_ctx *ctx, size_t height, size_t width, ien_spectral 
   sp->nba = (2 * h + 31) / 32;
   sp->nbx = (w + 31) / 32;
   const double s = 1.0 / std::sqrt((double)h * w);
+  const bool wide = h > MAX_SIDE || w > MAX_SIDE;
+  sp->wide = wide;
+  sp->scale = (float)s;
   // (cos, sin) of 2 pi j / n once each: a table asks for n^2 of them.
   const std::vector<double> trig_w = circle(w), trig_h = circle(h);
-  const int xp = sp->xp, yp = sp->yp;
+  const int xp = sp->xp, yp = sp->yp, yb = (h + 31) / 32;  // yb: blocks of 32 rows, steps of 16 folded ones
   // Row transform (A operand, rows m of R): cos for the real parts of
   // columns m < half, -sin for the imaginary parts of columns m - half + 1.
   const std::vector<uint16_t> tf = operand(sp->mb, 2 * xp / 16, [&](int m, int kk) -> uint16_t {
@@ -1188,40 +1295,47 @@ ien_status spectral_new(ien_ctx *ctx, size_t height, size_t width, ien_spectral 
     if (m >= w || x >= w) return 0;
     const int col = m < half ? m : m - half + 1;
     const double *t = &trig_w[2 * (col * x % w)];
-    return split_half(m < half ? t[0] : -t[1], term);
+    const double v = m < half ? t[0] : -t[1];
+    return wide ? split_scaled(v, term) : split_half(v, term);
   });
-  // Column transform (B operand, columns (part', ky)), x 1 / sqrt(h w) over R's scale:
-  // (a + i b) e^{-i theta}.  K: (term, part, y), terms hi, lo.
-  const std::vector<uint16_t> ta = operand(sp->nba, 4 * yp / 16, [&](int n, int kk) -> uint16_t {
+  // Column transform (B operand, columns (part', ky)), x 1 / sqrt(h w) x 64:
+  // (a + i b) e^{-i theta}.  K: (term, part, y), terms hi, lo.  Wide: columns
+  // ky, K: (cos or sin, piece, y < F) as k_spectral_tall folds them.
+  const std::vector<uint16_t> ta = wide ? operand(yb, 6 * yb, [&](int ky, int kk) -> uint16_t {
+    const int q = kk / (16 * yb), y = kk % (16 * yb);
+    if (ky >= h || y >= (h + 1) / 2) return 0;
+    const double *t = &trig_h[2 * (ky * y % h)];
+    const double v = q < 3 ? t[0] : y > 0 ? t[1] : h % 2 ? 0.0 : ky % 2 ? -1.0 : 1.0;
+    return split_bf16(v, 2 - q % 3);
+  }) : operand(sp->nba, 4 * yp / 16, [&](int n, int kk) -> uint16_t {
     const int term = kk / (2 * yp), part = (kk % (2 * yp)) / yp, y = kk % yp;
     if (n >= 2 * h || y >= h) return 0;
     const int pp = n / h, ky = n % h;
     const double c = trig_h[2 * (ky * y % h)], sn = trig_h[2 * (ky * y % h) + 1];
     const double v = pp == 0 ? (part == 0 ? c : sn) : (part == 0 ? -sn : c);
-    return split_half(v * s / r_scale(w), term);
+    return split_half(v * s * 64.0, term);
   });
   // Inverse columns (B operand, columns (part', y)): (a + i b) e^{+i theta}.
-  // K: (term, part, ky), terms hi, lo.
+  // K: (term, part, ky), terms hi, lo; wide: (part, term, ky).
   const std::vector<uint16_t> tc = operand(sp->nba, 4 * yp / 16, [&](int n, int kk) -> uint16_t {
-    const int term = kk / (2 * yp), part = (kk % (2 * yp)) / yp, ky = kk % yp;
+    const int q = kk / yp, ky = kk % yp;
     if (n >= 2 * h || ky >= h) return 0;
-    const int pp = n / h, y = n % h;
+    const int part = wide ? q / 2 : q % 2, pp = n / h, y = n % h;
     const double c = trig_h[2 * (ky * y % h)], sn = trig_h[2 * (ky * y % h) + 1];
     const double v = pp == 0 ? (part == 0 ? c : -sn) : (part == 0 ? sn : c);
-    return split_half(v, term);
+    return wide ? split_scaled(v, q % 2) : split_half(v, q / 2);
   });
-  // Inverse rows (B operand, columns x), x 1 / sqrt(h w) x 256: the real
-  // parts of column k times w_k cos, the imaginary parts times -w_k sin,
-  // w_k = 1 for column 0 and (even w) w / 2, else 2.  K: (term, m), terms
-  // hi, lo.
-  const std::vector<uint16_t> tr = operand(sp->nbx, 2 * xp / 16, [&](int x, int kk) -> uint16_t {
-    const int term = kk / xp, m = kk % xp;
+  // Inverse rows (B operand, pixels): x = w_k (re cos - im sin), w_k = 1 at
+  // k = 0 and (even w) k = w / 2, 2 elsewhere; the rows m of U as R's.  K:
+  // (term, m), terms hi, lo, / sqrt(h w) x 256; wide: (m / 16, term, m % 16).
+  const std::vector<uint16_t> tr = operand(sp->nbx, (wide ? 3 : 2) * xp / 16, [&](int x, int kk) -> uint16_t {
+    const int term = wide ? kk / 16 % 3 : kk / xp, m = wide ? kk / 48 * 16 + kk % 16 : kk % xp;
     if (x >= w || m >= w) return 0;
     const int col = m < half ? m : m - half + 1;
     const double wk = (col == 0 || 2 * col == w) ? 1.0 : 2.0;
     const double *t = &trig_w[2 * (col * x % w)];
     const double v = m < half ? wk * t[0] : -wk * t[1];
-    return split_half(v * s * 256.0, term);
+    return wide ? split_bf16(v, term) : split_half(v * s * 256.0, term);
   });
   auto put = [](uint16_t **d, const std::vector<uint16_t> &v) {
     hipError_t e = hipMalloc((void **)d, v.size() * 2);

@@ -1,0 +1,48 @@
+"""Internal functions of libien_hip.so that the tests call by their C++ names
+(no part of the C ABI: what they do is otherwise only reached through whole
+networks)."""
+
+import ctypes
+
+import ien
+
+_vp, _long, _int = ctypes.c_void_p, ctypes.c_long, ctypes.c_int
+
+
+def _function(name, *argtypes, restype=_int):
+    f = getattr(ien.load(), name)
+    f.argtypes, f.restype = argtypes, restype
+    return f
+
+
+def _ptr(t):
+    return None if t is None else t.data_ptr()
+
+
+class LongSpectral:
+    """lama.h spectral_new, _rows, _columns and _back: the fused spectral
+    branch of maps with sides up to 128, a launch group at a time."""
+
+    def __init__(self, ctx, height, width):
+        h = _vp()
+        new = _function("_ZN3ien12spectral_newEP7ien_ctxmmPP12ien_spectral", _vp, ctypes.c_size_t,
+                        ctypes.c_size_t, ctypes.POINTER(_vp))
+        ien.check(new(ctx.h, height, width, ctypes.byref(h)))
+        self.h = h
+
+    def rows(self, x, stride, m_in, spectral, r):
+        f = _function("_ZN3ien13spectral_rowsEPK12ien_spectralPKtlPK10ien_matrixPtPf", _vp, _vp, _long, _vp, _vp, _vp)
+        ien.check(f(self.h, _ptr(x), stride, m_in.h, _ptr(spectral), _ptr(r)))
+
+    def columns(self, m_f, r, z, u):
+        f = _function("_ZN3ien16spectral_columnsEPK12ien_spectralPK10ien_matrixPKfPtPf", _vp, _vp, _vp, _vp, _vp)
+        ien.check(f(self.h, m_f.h, _ptr(r), _ptr(z), _ptr(u)))
+
+    def back(self, m_out, spectral, u, out, stride, dst=None, add=None):
+        f = _function("_ZN3ien13spectral_backEPK12ien_spectralPK10ien_matrixPKtPKfPtlSA_S7_", _vp, _vp, _vp, _vp, _vp,
+                      _long, _vp, _vp)
+        ien.check(f(self.h, m_out.h, _ptr(spectral), _ptr(u), _ptr(out), stride, _ptr(dst), _ptr(add)))
+
+    def free(self):
+        ien.load().ien_spectral_free(self.h)
+        self.h = None
