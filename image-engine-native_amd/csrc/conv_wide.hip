@@ -404,6 +404,14 @@ ien_status launch_wide(ien_ctx *ctx, const ConvArgs &a, const WidePlan &plan) {
   }
 }
 
+// Input bytes up to the padding loads' out-of-range offset, outputs in 31 bits
+// of elements: every map that LaMa's first convolution can write at full scale
+// (2^31 values of 64 channels) comes up again.
+bool conv_up_fits(long h, long w, long c, long n, long ys) {
+  return h > 0 && w > 0 && c > 0 && c % 64 == 0 && n > 0 && n % 8 == 0 && ys % 8 == 0 && ys >= n &&
+         h * w * c * 2 <= OOB && 4 * h * w * ys < (1L << 31);
+}
+
 // LaMa's doublings (1000 x 680 images, us): 85 x 125, 512 -> 256 as four
 // launches of the general kernel 112, here 43; 170 x 250, 256 -> 128 112 and
 // 48; 340 x 500, 128 -> 64 110 and 57.
@@ -420,9 +428,7 @@ ien_status conv_up(ien_ctx *ctx, const uint16_t *x, int h, int w, int c, ien_mat
     up.bias[p] = phases[p]->d_bias;
     up.kb[p] = phases[p]->kb;
   }
-  IEN_CHECK(c % 64 == 0 && n % 8 == 0 && ys % 8 == 0 && ys >= n && (((uintptr_t)x | (uintptr_t)y) & 15) == 0 &&
-                (long)h * w * c * 2 <= 0x7fff0000L && 4L * h * w * ys < (1L << 31),
-            IEN_ERR_INPUT, "doubling of a %d x %d map, %d -> %d channels", w, h, c, n);
+  IEN_CHECK(conv_up_fits(h, w, c, n, ys) && (((uintptr_t)x | (uintptr_t)y) & 15) == 0, IEN_ERR_INPUT, "doubling of a %d x %d map, %d -> %d channels", w, h, c, n);
   ConvArgs a{};
   a.x = x;
   a.H = a.OH = h;

@@ -189,6 +189,8 @@ ien_status launch_conv(ien_ctx *ctx, const ConvCall &c);
 // pixels c apart), each result stored at its pixel of the 2h x 2w map y.
 ien_status conv_up(ien_ctx *ctx, const uint16_t *x, int h, int w, int c, ien_matrix *const *phases, uint16_t *y,
                    int ys, ien_act act);
+// The maps it takes, by their sizes.
+bool conv_up_fits(long h, long w, long c, long n, long ys);
 
 // conv_pair.hip: two 3x3 64 -> 64 convolutions with bias and PReLU in one
 // launch (x -> w1 -> w2 -> y, the intermediate map never stored): NHWC f16

@@ -46,3 +46,16 @@ class LongSpectral:
     def free(self):
         ien.load().ien_spectral_free(self.h)
         self.h = None
+
+
+def conv_up_fits(h, w, c, n, ys):
+    f = _function("_ZN3ien12conv_up_fitsElllll", *[_long] * 5, restype=ctypes.c_bool)
+    return f(h, w, c, n, ys)
+
+
+def conv_up(ctx, x, h, w, c, phases, y, ys, act):
+    """ien_internal.h conv_up: a doubling's four phases in one launch."""
+    f = _function("_ZN3ien7conv_upEP7ien_ctxPKtiiiPKP10ien_matrixPti7ien_act", _vp, _vp, _int, _int, _int,
+                  ctypes.POINTER(_vp), _vp, _int, _int)
+    handles = (_vp * 4)(*[m.h for m in phases])
+    ien.check(f(ctx.h, _ptr(x), h, w, c, handles, _ptr(y), ys, act))
