@@ -418,6 +418,7 @@ bool conv_up_fits(long h, long w, long c, long n, long ys) {
 ien_status conv_up(ien_ctx *ctx, const uint16_t *x, int h, int w, int c, ien_matrix *const *phases, uint16_t *y,
                    int ys, ien_act act) {
   const int n = (int)phases[0]->n;
+  IEN_CHECK(act != IEN_ACT_PRELU, IEN_ERR_INPUT, "a doubling takes no slopes");
   UpWeights up{};
   for (int p = 0; p < 4; p++) {
     const int taps = (1 + p / 2) * (1 + p % 2);

@@ -186,7 +186,8 @@ ien_status launch_conv(ien_ctx *ctx, const ConvCall &c);
 // conv_wide.hip: the four phases of a doubling transposed 3 x 3 convolution
 // (phase 2 py + px reads pixel (y, x) and, where py or px is set, the next one
 // down or across, taps in row order) over an h x w map of c channels (64s,
-// pixels c apart), each result stored at its pixel of the 2h x 2w map y.
+// pixels c apart), each result stored at its pixel of the 2h x 2w map y.  Any
+// activation but PReLU.
 ien_status conv_up(ien_ctx *ctx, const uint16_t *x, int h, int w, int c, ien_matrix *const *phases, uint16_t *y,
                    int ys, ien_act act);
 // The maps it takes, by their sizes.

@@ -54,6 +54,18 @@ def test_doubling_matches_its_phases(ctx, h, w, c, n, pad, act):
     compare(ctx, x, h, w, c, n, phases_of(ctx, c, n, rng), n + pad, act)
 
 
+def test_doubling_refuses_prelu(ctx):
+    import ien
+    import torch
+
+    rng = np.random.default_rng(2)
+    x = torch.zeros((2, 2, 64), dtype=torch.float16, device="cuda")
+    y = torch.zeros((4, 4, 8), dtype=torch.float16, device="cuda")
+    with pytest.raises(ien.IenError) as e:
+        conv_up(ctx, x, 2, 2, 64, phases_of(ctx, 64, 8, rng), y, 8, ien.ACT_PRELU)
+    assert e.value.status == ien.ERR_INPUT
+
+
 def test_doubling_of_the_largest_map(ctx):
     """The last doubling of a 6384 x 5256 image (33 554 304 padded pixels): an
     input of 2^31 - 2^13 bytes, outputs of 2^31 - 2^13 values."""
