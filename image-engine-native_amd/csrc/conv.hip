@@ -1217,16 +1217,21 @@ static int pick_ck(int c) { return c % 64 == 0 ? 64 : c % 32 == 0 ? 32 : 16; }
 // 64 x 96, 256 -> 256 14.5; 85 x 125, 512 -> 128 25.5; 128 x 192, 128 -> 128
 // 12.8; 95 x 95, 512 -> 256 34; 85 x 125, 128 -> 384 19.7; 71 x 472,
 // 512 -> 128 65; 200 x 200, 256 -> 256 70).
-static double general_us(const ien_ctx *ctx, const ConvArgs &a) {
-  const long tiles = (long)((a.OH + 3) / 4) * ((a.OW + 31) / 32) * ((a.N + 63) / 64);
-  const int chunks = a.C / 32;
-  const double round = (double)tiles / ctx->cus;
+static double general_us(int cus, int ow, int c, int n, long p_begin, long p_end) {
+  const long tiles = range_tiles(ow, p_begin, p_end, n, 4, 64);
+  const int chunks = c / 32;
+  const double round = (double)tiles / cus;
   if (round <= 1) {
-    const int splits = round <= 0.25 ? (int)std::min<long>(chunks / 2, ctx->cus / tiles) : 1;
+    const int splits = round <= 0.25 ? (int)std::min<long>(chunks / 2, cus / tiles) : 1;
     return splits > 1 ? 8.5 + 1.2 * ((chunks + splits - 1) / splits) : 5.5 + 1.2 * chunks;
   }
   if (round <= 2) return 5.4 + 1.85 * chunks;
   return 4.6 + chunks * std::max(3.78, 1.5 * round);
+}
+
+int conv3_choice(int cus, long workspace, int ow, int c, int n, long p_begin, long p_end) {
+  const WidePlan plan = wide_plan(cus, workspace, ow, c, n, p_begin, p_end);
+  return plan.us < general_us(cus, ow, c, n, p_begin, p_end) ? 16 * plan.tile + plan.ksplit : -1;
 }
 
 ien_status launch_conv(ien_ctx *ctx, const ConvCall &c) {
@@ -1340,9 +1345,9 @@ ien_status launch_conv(ien_ctx *ctx, const ConvCall &c) {
     }
     // 64s of channels: the pipelined kernel of a workgroup a CU, where it is
     // estimated to be the faster one.
-    if (!nchw && ck == 64) {
-      const WidePlan plan = wide_plan(ctx, a);
-      if (plan.us > 0 && plan.us < general_us(ctx, a)) return launch_wide(ctx, a, plan);
+    if (!nchw && ck == 64 && wide_supported(ctx, a)) {
+      const int choice = conv3_choice(ctx->cus, (long)ctx->splitk_floats, a.OW, a.C, a.N, a.p_begin, a.p_end);
+      if (choice >= 0) return launch_wide(ctx, a, choice / 16, choice % 16);
     }
     // NHWC: 4 x 32 tiles and 32-channel chunks, so that the halo and weight
     // stages of three workgroups fit a CU's LDS and hide each other's load

@@ -326,16 +326,29 @@ ien_status launch_narrow(ien_ctx *ctx, ConvArgs a, int ks);
 bool few_supported(const ConvArgs &a, int ks, int stride, int nchw, int noff, int rows_mode);
 ien_status launch_few(ien_ctx *ctx, ConvArgs a, int ks);
 
+// Tiles of `rows` x 32 pixels x `cols` channels that hold output pixels
+// p_begin .. p_end - 1 of a map `ow` wide, of n channels: what a launch over
+// that range runs, and what a choice between launches has to count.
+inline long range_tiles(int ow, long p_begin, long p_end, int n, int rows, int cols) {
+  return ((p_end - 1) / ow / rows + 1 - p_begin / ow / rows) * ((ow + 31) / 32) * ((n + cols - 1) / cols);
+}
+
 // conv_wide.hip: 3 x 3 stride-1 NHWC convolutions of 64s of channels with f16
-// outputs in 16-byte groups.
-// The estimated microseconds (of the best tile and split), or a
-// negative number where the kernel does not serve.
+// outputs in 16-byte groups.  Whether the kernel serves; its best tile and
+// split for a range of pixels, with the microseconds they are estimated at.
+bool wide_supported(const ien_ctx *ctx, const ConvArgs &a);
 struct WidePlan {
   double us;
   int tile, ksplit;
 };
-WidePlan wide_plan(const ien_ctx *ctx, const ConvArgs &a);
-ien_status launch_wide(ien_ctx *ctx, const ConvArgs &a, const WidePlan &plan);
+WidePlan wide_plan(int cus, long workspace, int ow, int c, int n, long p_begin, long p_end);
+ien_status launch_wide(ien_ctx *ctx, const ConvArgs &a, int tile, int ksplit);
+
+// conv.hip: the kernel of a 3 x 3 NHWC convolution over pixels p_begin ..
+// p_end - 1 of a map ow wide, c -> n channels, on a device of `cus` CUs with a
+// workspace of `workspace` floats.  Stride 1, 64s of channels, where conv_wide
+// serves: 16 x its tile + its split, or -1 for the general kernel.
+int conv3_choice(int cus, long workspace, int ow, int c, int n, long p_begin, long p_end);
 
 // conv_nchw.hip: 1x1 products of whole NCHW f16 planes into NCHW f16
 // planes (pixels a multiple of 8, 16-byte aligned planes), not accumulating.

@@ -374,20 +374,21 @@ constexpr double SPLIT_US = 6.0;
 // 512 -> 256 34 -> 28 (8 x 64); and, left to the general kernel's deep
 // splits, 64 x 64, 512 -> 128 14.4 against 17.9.  Not compact launches: a workgroup leaves
 // another branch's kernels no LDS.
-WidePlan wide_plan(const ien_ctx *ctx, const ConvArgs &a) {
+bool wide_supported(const ien_ctx *ctx, const ConvArgs &a) {
+  return a.C % 64 == 0 && a.N % 8 == 0 && a.ys % 8 == 0 && (((uintptr_t)a.y | (uintptr_t)a.add2) & 15) == 0 &&
+         !a.out_nchw && !a.out_f32 && !ctx->compact && (long)a.H * a.W * a.xs * 2 <= 0x7fff0000L &&
+         (long)a.NB * a.KB * 1024 <= 0x7fff0000L;
+}
+
+WidePlan wide_plan(int cus, long workspace, int ow, int c, int n, long p_begin, long p_end) {
   WidePlan best{-1.0, 0, 1};
-  if (a.C % 64 || a.N % 8 || a.ys % 8 || (((uintptr_t)a.y | (uintptr_t)a.add2) & 15) || a.out_nchw ||
-      a.out_f32 || ctx->compact || (long)a.H * a.W * a.xs * 2 > 0x7fff0000L ||
-      (long)a.NB * a.KB * 1024 > 0x7fff0000L)
-    return best;
-  const int chunks = a.C / 64;
-  const int row0 = a.p_begin / a.OW, row1 = (a.p_end - 1) / a.OW;
+  const int chunks = c / 64;
   for (int i = 0; i < (int)(sizeof TILES / sizeof TILES[0]); i++) {
     const Tile &t = TILES[i];
-    const long blocks = (long)(row1 / t.rows + 1 - row0 / t.rows) * ((a.OW + 31) / 32) * ((a.N + t.cols - 1) / t.cols);
+    const long blocks = range_tiles(ow, p_begin, p_end, n, t.rows, t.cols);
     for (int s = 1; s <= 4 && s <= chunks; s++) {
-      if (s > 1 && (!t.sums || blocks > ien_ctx::SPLITK_TILES || blocks * s * t.sums > (long)ctx->splitk_floats)) break;
-      const double rounds = (double)((blocks * s + ctx->cus - 1) / ctx->cus);
+      if (s > 1 && (!t.sums || blocks > ien_ctx::SPLITK_TILES || blocks * s * t.sums > workspace)) break;
+      const double rounds = (double)((blocks * s + cus - 1) / cus);
       const double us = rounds * (t.round + t.chunk * ((chunks + s - 1) / s)) + (s > 1 ? SPLIT_US : 0.0);
       if (best.us < 0 || us < best.us) best = WidePlan{us, i, s};
     }
@@ -395,11 +396,11 @@ WidePlan wide_plan(const ien_ctx *ctx, const ConvArgs &a) {
   return best;
 }
 
-ien_status launch_wide(ien_ctx *ctx, const ConvArgs &a, const WidePlan &plan) {
-  switch (plan.tile) {
-    case 0: return launch<8, 1, 1, 8>(ctx, a, plan.ksplit);
-    case 1: return launch<4, 2, 1, 6>(ctx, a, plan.ksplit);
-    case 2: return launch<8, 2, 1, 4>(ctx, a, plan.ksplit);
+ien_status launch_wide(ien_ctx *ctx, const ConvArgs &a, int tile, int ksplit) {
+  switch (tile) {
+    case 0: return launch<8, 1, 1, 8>(ctx, a, ksplit);
+    case 1: return launch<4, 2, 1, 6>(ctx, a, ksplit);
+    case 2: return launch<8, 2, 1, 4>(ctx, a, ksplit);
     default: return launch<4, 1, 2, 8>(ctx, a, 1);
   }
 }

@@ -59,3 +59,10 @@ def conv_up(ctx, x, h, w, c, phases, y, ys, act):
                   ctypes.POINTER(_vp), _vp, _int, _int)
     handles = (_vp * 4)(*[m.h for m in phases])
     ien.check(f(ctx.h, _ptr(x), h, w, c, handles, _ptr(y), ys, act))
+
+
+def conv3_choice(cus, workspace, ow, c, n, p_begin, p_end):
+    """conv_common.h conv3_choice: (tile, split) of conv_wide, or None."""
+    f = _function("_ZN3ien12conv3_choiceEiliiill", _int, _long, _int, _int, _int, _long, _long)
+    r = f(cus, workspace, ow, c, n, p_begin, p_end)
+    return None if r < 0 else (r // 16, r % 16)

@@ -1,8 +1,11 @@
-"""The sizes that the convolution kernels accept (host code, no GPU)."""
+"""The sizes that the convolution kernels accept, and which of them a size
+takes (host code, no GPU)."""
 
 import pytest
 
-from internal import conv_up_fits
+from internal import conv3_choice, conv_up_fits
+
+CUS, WORKSPACE = 256, 8 << 20  # MI355X; the context's workspace in floats
 
 
 # LaMa's maps at P padded pixels: 64 channels at full scale, 128, 256 and 512
@@ -20,3 +23,31 @@ def test_doublings_take_every_map_that_fits_the_first_convolution(pixels, fits):
                                         (4, 4, 64, 64, 56), (4, 4, 64, 64, 68)])
 def test_doublings_refuse_other_layouts(h, w, c, n, ys):
     assert not conv_up_fits(h, w, c, n, ys)
+
+
+# conv_wide's tiles in order: 8 x 64, 4 x 128, 8 x 128, 4 x 64 (rows x
+# channels, 32 pixels wide).  The sizes of test_gpu_conv's test_conv3x3_wide
+# and its splits, which are there for the tile named here.
+@pytest.mark.parametrize("h,w,c,n,row0,rows,want", [
+    (85, 125, 512, 128, 0, None, (3, 1)), (61, 67, 384, 136, 0, None, (3, 1)), (70, 77, 512, 128, 0, None, (0, 4)),
+    (95, 95, 512, 232, 0, None, (1, 1)), (131, 163, 128, 200, 0, None, (2, 1)), (253, 250, 128, 64, 700, 62001, (0, 1)),
+    (2, 4000, 512, 128, 0, None, (3, 1)), (2500, 3, 192, 128, 0, None, (1, 1)),
+    (40, 200, 512, 128, 0, None, (1, 3)), (73, 200, 768, 120, 0, None, (2, 3)), (49, 200, 1024, 128, 0, None, (1, 2)),
+    (64, 64, 512, 128, 0, None, None)])
+def test_wide_tiles(h, w, c, n, row0, rows, want):
+    assert conv3_choice(CUS, WORKSPACE, w, c, n, row0, row0 + (h * w if rows is None else rows)) == want
+
+
+# A band of a tall map is the work of a map of its own height: 4 rows of 1000 x
+# 64 pixels, 512 -> 128, took 15.0 us on the tiles that suit the whole map, 10.2
+# on the general kernel's splits.
+@pytest.mark.parametrize("w,c,n", [(64, 512, 128), (95, 512, 256), (125, 512, 128), (300, 256, 256), (512, 128, 128)])
+@pytest.mark.parametrize("first,rows", [(0, 4), (8, 4), (480, 8), (96, 20), (16, 40), (800, 100)])
+def test_bands_choose_by_their_own_rows(w, c, n, first, rows):
+    assert conv3_choice(CUS, WORKSPACE, w, c, n, first * w, (first + rows) * w) == \
+        conv3_choice(CUS, WORKSPACE, w, c, n, 0, rows * w)
+
+
+def test_a_narrow_band_keeps_the_general_kernels_splits():
+    assert conv3_choice(CUS, WORKSPACE, 64, 512, 128, 500 * 64, 504 * 64) is None
+    assert conv3_choice(CUS, WORKSPACE, 64, 512, 128, 0, 1000 * 64) is not None

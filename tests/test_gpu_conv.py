@@ -150,6 +150,15 @@ def test_conv3x3_wide(ctx, oracle, h, w, c, n, pad, act, acc, row0, rows, sp):
     assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
 
 
+# Splits of 4 x 128 and 8 x 128 tiles, and a band of a tall map: rows that start
+# and end within a tile, on the general kernel's splits.
+@pytest.mark.parametrize("h,w,c,n,pad,act,acc,row0,rows,sp", [
+    (40, 200, 512, 128, 1, 1, False, 0, None, 0), (73, 200, 768, 120, 0, 0, True, 0, None, 8),
+    (400, 64, 512, 128, 0, 1, False, 199 * 64 + 5, 300, 0), (400, 64, 512, 128, 1, 0, True, 130 * 64, 100 * 64, 0)])
+def test_conv3x3_wide_splits_and_bands(ctx, oracle, h, w, c, n, pad, act, acc, row0, rows, sp):
+    test_conv3x3_wide(ctx, oracle, h, w, c, n, pad, act, acc, row0, rows, sp)
+
+
 @pytest.mark.parametrize("c", [3, 4, 8, 16])
 def test_conv3x3_few_channels(ctx, oracle, c):
     x, wt, b = case(2, 11, 37, c, 64, 9)
