@@ -1234,6 +1234,16 @@ int conv3_choice(int cus, long workspace, int ow, int c, int n, long p_begin, lo
   return plan.us < general_us(cus, ow, c, n, p_begin, p_end) ? 16 * plan.tile + plan.ksplit : -1;
 }
 
+// 32-channel chunks where a CU gets at most one tile of the range
+// (double-buffered: 128 x 128, 256 -> 512 19.1 us, 21.6 with 16); over that
+// 16-channel ones, whose halo and weights leave room for four workgroups a CU
+// instead of two (us, 32 -> 16: 680 x 1000, 64 -> 128 69.6 -> 57.6; 340 x 500,
+// 128 -> 256 60.7 -> 54.7; 170 x 250, 256 -> 512 74.9 -> 54.9; 512 x 512,
+// 64 -> 128 26.7 -> 24.4).
+int stride2_choice(int cus, int ow, int n, long p_begin, long p_end) {
+  return range_tiles(ow, p_begin, p_end, n, 4, 64) <= cus ? 32 : 16;
+}
+
 ien_status launch_conv(ien_ctx *ctx, const ConvCall &c) {
   const ien_matrix *w = c.w;
   IEN_CHECK(w && w->d_packed, IEN_ERR_INPUT, "no weights");
@@ -1372,14 +1382,8 @@ ien_status launch_conv(ien_ctx *ctx, const ConvCall &c) {
   if (c.ks == 3 && c.stride == 2) {
     IEN_CHECK(!nchw, IEN_ERR_INPUT, "strided convolutions read NHWC");
     if (!vec) return run_cfg<3, 2, 4, 32, 4, 2, 16, false, false>(ctx, a);
-    // 32-channel chunks where a CU gets at most one tile (double-buffered:
-    // 128 x 128, 256 -> 512 19.1 us, 21.6 with 16); over that 16-channel ones,
-    // whose halo and weights leave room for four workgroups a CU instead of
-    // two (us, 32 -> 16: 680 x 1000, 64 -> 128 69.6 -> 57.6; 340 x 500,
-    // 128 -> 256 60.7 -> 54.7; 170 x 250, 256 -> 512 74.9 -> 54.9; 512 x 512,
-    // 64 -> 128 26.7 -> 24.4).
-    const long tiles = (long)((c.OH + 3) / 4) * ((c.OW + 31) / 32) * ((w->n + 63) / 64);
-    if (ck >= 32 && tiles <= ctx->cus) return run_cfg<3, 2, 4, 32, 4, 2, 32, true, false>(ctx, a);
+    if (ck >= 32 && stride2_choice(ctx->cus, a.OW, a.N, a.p_begin, a.p_end) == 32)
+      return run_cfg<3, 2, 4, 32, 4, 2, 32, true, false>(ctx, a);
     return run_cfg<3, 2, 4, 32, 4, 2, 16, true, false>(ctx, a);
   }
   if (c.ks == 1 && c.stride == 1) {

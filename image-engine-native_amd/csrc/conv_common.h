@@ -347,8 +347,10 @@ ien_status launch_wide(ien_ctx *ctx, const ConvArgs &a, int tile, int ksplit);
 // conv.hip: the kernel of a 3 x 3 NHWC convolution over pixels p_begin ..
 // p_end - 1 of a map ow wide, c -> n channels, on a device of `cus` CUs with a
 // workspace of `workspace` floats.  Stride 1, 64s of channels, where conv_wide
-// serves: 16 x its tile + its split, or -1 for the general kernel.
+// serves: 16 x its tile + its split, or -1 for the general kernel.  Stride 2,
+// 32s of channels: the general kernel's channels a chunk.
 int conv3_choice(int cus, long workspace, int ow, int c, int n, long p_begin, long p_end);
+int stride2_choice(int cus, int ow, int n, long p_begin, long p_end);
 
 // conv_nchw.hip: 1x1 products of whole NCHW f16 planes into NCHW f16
 // planes (pixels a multiple of 8, 16-byte aligned planes), not accumulating.

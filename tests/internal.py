@@ -66,3 +66,9 @@ def conv3_choice(cus, workspace, ow, c, n, p_begin, p_end):
     f = _function("_ZN3ien12conv3_choiceEiliiill", _int, _long, _int, _int, _int, _long, _long)
     r = f(cus, workspace, ow, c, n, p_begin, p_end)
     return None if r < 0 else (r // 16, r % 16)
+
+
+def stride2_choice(cus, ow, n, p_begin, p_end):
+    """conv_common.h stride2_choice: the general kernel's channels a chunk."""
+    f = _function("_ZN3ien14stride2_choiceEiiill", _int, _int, _int, _long, _long)
+    return f(cus, ow, n, p_begin, p_end)

@@ -317,6 +317,14 @@ def test_stride2_large_grid(ctx, oracle, h, w, c, n, pad):
     close(run_gpu(ctx, x, wt, b, step=2, pad=pad, act=1), want_cpu(oracle, x, wt, b, step=2, pad=pad, act=1))
 
 
+# A band of it, within a tile at either end.
+def test_stride2_band(ctx, oracle):
+    x, wt, b = case(31, 257, 511, 64, 128, 9)
+    row0, rows = 40 * 256 + 7, 21 * 256
+    want = want_cpu(oracle, x, wt, b, step=2, act=1)
+    close(run_gpu(ctx, x, wt, b, step=2, act=1, row0=row0, rows=rows), want[row0:row0 + rows])
+
+
 def test_reflect_3x3(ctx, oracle):
     x, wt, b = case(8, 9, 70, 64, 64, 9)
     close(run_gpu(ctx, x, wt, b, pad=1), want_cpu(oracle, x, wt, b, pad=1))
