@@ -310,6 +310,9 @@ ien_status splitk_finish(ien_ctx *ctx, int ksplit, long rows, int pitch, const C
 // the chip.
 bool rows_supported(const ConvArgs &a, long rows);
 ien_status launch_rows(ien_ctx *ctx, const ConvArgs &a);
+// How it runs m rows, k -> n, on a device of `cus` CUs with a workspace of
+// `workspace` floats: in this many splits, negative for eight waves a tile.
+int rows_choice(int cus, long workspace, int m, int k, int n);
 
 // conv_res.hip: the resident-weight kernel for NHWC inputs of 16, 32 or 64
 // channels with k x k (k = 1, 3) zero-padded taps and K = k k C <= 640.

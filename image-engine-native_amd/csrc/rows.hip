@@ -25,7 +25,7 @@
 //    gemm.rs:583-666.
 // Chunks of 32 channels keep the ring at 36 KiB (64 x 128 tiles), so several
 // workgroups share a CU and hide each other's latency.
-// Where the tiles leave no CU a second workgroup (KG = 2) nothing hides the
+// Where the tiles leave no CU a second workgroup (KG = 2; rows_plan) nothing hides the
 // latency of four waves that wait for a chunk, read its fragments and
 // multiply them in turn (a 32-deep chunk took some 0.18 us, 0.05 of them
 // products).  There eight waves take a tile: chunks are 64 deep, each set of
@@ -415,39 +415,52 @@ __global__ __launch_bounds__(256 * KG) void k_rows(RowsArgs a) {
   }
 }
 
-// Eight waves a tile where a CU gets at most one of them (see above), in
-// whole 64-deep chunks of one plane or pixel.
-template <int BM, int MODE>
-bool paired(const ien_ctx *ctx, const RowsArgs &a) {
-  return BM == 64 && a.tiles <= ctx->cus && a.K % 64 == 0 && a.k1 % 64 == 0 && (MODE != 1 || a.K % 256 == 0);
-}
+struct RowsPlan {
+  bool eight;
+  int ksplit;
+};
 
+// Eight waves a tile where a CU gets at most one of them (see above), in 64-deep
+// chunks (`whole`: each lies in one plane or pixel) and with four of them or
+// more: below that four waves, several tiles a CU, are the faster ones (us,
+// four waves -> eight: 3951 x 64 -> 192 4.2 -> 4.7, 8000 x 192 -> 256 5.5 ->
+// 6.0, 900 x 128 -> 128 4.5 -> 4.6; 1762 x 256 -> 520 5.7 -> 5.5, 8000 x 384
+// -> 256 7.0 -> 6.5).
+//
 // Split-K when the tiles leave three quarters of the CUs idle: about two
 // workgroups per CU, each split at least 256 deep, where that is estimated
 // to be faster.  A split launch and its finishing pass take some 7.5 us and
 // 2.4 more a million partial sums (100 x 4096 -> 256 8.6 us; 256 x 3072 -> 768
 // 14.0, 512 x 2048 -> 512 12.9, 949 x 2048 -> 512 17); one launch of eight
 // waves a tile 4.2 and 0.27 a 64-deep chunk (21.0, 17.2, 12.6, 13.0).
+RowsPlan rows_plan(int cus, long workspace, int m, int k, int n, int bm, int bn, bool whole, bool split) {
+  const int tiles_n = (n + bn - 1) / bn, tiles = (m + bm - 1) / bm * tiles_n, chunks = k / 32;
+  const long sums = (long)m * tiles_n * bn;
+  RowsPlan p{bm == 64 && whole && tiles <= cus && k >= 256 && k % 64 == 0, 1};
+  if (split && chunks >= 16 && 4 * tiles <= cus) {
+    p.ksplit = std::min(chunks / 8, (2 * cus + tiles - 1) / tiles);
+    while (p.ksplit > 1 && p.ksplit * sums > workspace) p.ksplit--;
+  }
+  if (p.eight && p.ksplit > 1) {
+    p.eight = 4.2 + 0.27 * (k / 64) < 7.5 + 2.4e-6 * p.ksplit * sums;
+    if (p.eight) p.ksplit = 1;
+  }
+  return p;
+}
+
 template <int BM, int BN, int KC, int MODE = 0>
 ien_status launch(ien_ctx *ctx, RowsArgs a, const ConvArgs &c) {
   a.tiles_n = (a.N + BN - 1) / BN;
   a.tiles = (a.M + BM - 1) / BM * a.tiles_n;
-  int chunks = a.K / KC;
   a.pitch = a.tiles_n * BN;
-  int ksplit = 1;
   // (The finishing pass writes one map, row by row; gathered rows are
   // split like any others.)
   const bool planes = a.k1 < a.K || a.n1 < a.N || MODE >= 2;
-  if (!planes && chunks >= 16 && 4 * a.tiles <= ctx->cus) {
-    ksplit = std::min(chunks / 8, (2 * ctx->cus + a.tiles - 1) / a.tiles);
-    while (ksplit > 1 && (size_t)ksplit * a.M * a.pitch > ctx->splitk_floats) ksplit--;
-  }
-  bool pair = paired<BM, MODE>(ctx, a);
-  if (pair && ksplit > 1) {
-    pair = 4.2 + 0.27 * (a.K / 64) < 7.5 + 2.4e-6 * ksplit * a.M * a.pitch;
-    if (pair) ksplit = 1;
-  }
-  if (pair) chunks = a.K / 64;
+  const RowsPlan plan = rows_plan(ctx->cus, (long)ctx->splitk_floats, a.M, a.K, a.N, BM, BN,
+                                  a.k1 % 64 == 0 && (MODE != 1 || a.K % 256 == 0), !planes);
+  const bool pair = plan.eight;
+  const int chunks = a.K / (pair ? 64 : KC);
+  int ksplit = plan.ksplit;
   a.kchunks = (chunks + ksplit - 1) / ksplit;
   ksplit = (chunks + a.kchunks - 1) / a.kchunks;
   a.part = ksplit > 1 ? ctx->splitk : nullptr;
@@ -470,9 +483,9 @@ ien_status launch(ien_ctx *ctx, RowsArgs a, const ConvArgs &c) {
 
 static long tiles_of(long rows, int bm, int n) { return (rows + bm - 1) / bm * ((n + 127) / 128); }
 
-// Any number of tiles that eight waves each can take (64s of channels: 104 x
-// 384 -> 384 7.4 us on the general kernel, 5.8 here; 145 x 1024 -> 256 10.4
-// and 8.4; 900 x 128 -> 128 5.4 and 5.0); else 128-row tiles when they number
+// Any number of tiles of 64s of channels (104 x 384 -> 384 7.4 us on the
+// general kernel, 5.8 here; 145 x 1024 -> 256 10.4 and 8.4; 900 x 128 -> 128
+// 5.4 and 4.5); else 128-row tiles when they number
 // at least 128, 64-row tiles when those number at least 96, or at least 8
 // with K 512 deep (split-K); below that the general kernel serves.
 bool rows_supported(const ConvArgs &a, long rows) {
@@ -486,6 +499,14 @@ bool rows_supported(const ConvArgs &a, long rows) {
 
 // Rows p_begin .. p_end of x (row stride xs) times the packed weights into
 // rows 0 .. of y; a.C is the reduction depth.
+static bool rows_narrow(int m, int n) { return n <= 64 && tiles_of(m, 128, n) >= 128; }
+
+int rows_choice(int cus, long workspace, int m, int k, int n) {
+  const bool narrow = rows_narrow(m, n);
+  const RowsPlan p = rows_plan(cus, workspace, m, k, n, narrow ? 128 : 64, narrow ? 64 : 128, true, true);
+  return p.eight ? -p.ksplit : p.ksplit;
+}
+
 ien_status launch_rows(ien_ctx *ctx, const ConvArgs &c) {
   RowsArgs a{};
   a.x = c.x + (long)c.p_begin * c.xs;
@@ -511,7 +532,7 @@ ien_status launch_rows(ien_ctx *ctx, const ConvArgs &c) {
   // Columns over 64: 64-row tiles (four workgroups a CU, twice the tiles of
   // 128-row ones; measured faster on every model shape); up to 64 columns:
   // 128 x 64 tiles.
-  if (c.N > 64 || tiles_of(a.M, 128, a.N) < 128) return launch<64, 128, 32>(ctx, a, c);
+  if (!rows_narrow(a.M, a.N)) return launch<64, 128, 32>(ctx, a, c);
   return launch<128, 64, 32>(ctx, a, c);
 }
 

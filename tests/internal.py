@@ -72,3 +72,9 @@ def stride2_choice(cus, ow, n, p_begin, p_end):
     """conv_common.h stride2_choice: the general kernel's channels a chunk."""
     f = _function("_ZN3ien14stride2_choiceEiiill", _int, _int, _int, _long, _long)
     return f(cus, ow, n, p_begin, p_end)
+
+
+def rows_choice(cus, workspace, m, k, n):
+    """conv_common.h rows_choice: (waves a tile, splits)."""
+    r = _function("_ZN3ien11rows_choiceEiliii", _int, _long, _int, _int, _int)(cus, workspace, m, k, n)
+    return 8 if r < 0 else 4, abs(r)

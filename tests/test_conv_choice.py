@@ -1,9 +1,9 @@
-"""The sizes that the convolution kernels accept, and which of them a size
-takes (host code, no GPU)."""
+"""The sizes that the convolution and row-product kernels accept, and which of
+them a size takes (host code, no GPU)."""
 
 import pytest
 
-from internal import conv3_choice, conv_up_fits, stride2_choice
+from internal import conv3_choice, conv_up_fits, rows_choice, stride2_choice
 
 CUS, WORKSPACE = 256, 8 << 20  # MI355X; the context's workspace in floats
 
@@ -63,3 +63,21 @@ def test_stride2_bands_choose_by_their_own_rows():
     assert stride2_choice(CUS, 256, 64, 0, 128 * 256) == 32
     assert stride2_choice(CUS, 256, 64, 0, 128 * 256 + 1) == 16
     assert stride2_choice(CUS, 256, 64, 2 * 256, 130 * 256) == 16
+
+
+# Products of few channels keep four waves a tile: eight, which wait for no
+# other workgroup, lose on three 64-deep chunks and less (3951 x 64 -> 192 4.2
+# us on four, 4.7 on eight).
+@pytest.mark.parametrize("m,n", [(1, 8), (900, 128), (1762, 520), (3951, 192), (8000, 256), (8192, 256)])
+def test_shallow_products_keep_four_waves(m, n):
+    for k in (64, 128, 192):
+        assert rows_choice(CUS, WORKSPACE, m, k, n) == (4, 1)
+    for k in (256, 384, 448):
+        assert rows_choice(CUS, WORKSPACE, m, k, n) == (8, 1)
+    assert rows_choice(CUS, WORKSPACE, m, 288, n) == (4, 1)  # (not whole 64-deep chunks)
+
+
+def test_more_tiles_than_cus_keep_four_waves():
+    assert rows_choice(CUS, WORKSPACE, 8193, 384, 256) == (4, 1)
+    assert rows_choice(CUS, WORKSPACE, 64 * 257, 1536, 128) == (4, 1)
+    assert rows_choice(CUS, WORKSPACE, 128 * 128, 1536, 64) == (4, 1)  # 128-row tiles
