@@ -427,25 +427,32 @@ struct RowsPlan {
 // 6.0, 900 x 128 -> 128 4.5 -> 4.6; 1762 x 256 -> 520 5.7 -> 5.5, 8000 x 384
 // -> 256 7.0 -> 6.5).
 //
-// Split-K when the tiles leave three quarters of the CUs idle: about two
-// workgroups per CU, each split at least 256 deep, where that is estimated
-// to be faster.  A split launch and its finishing pass take some 7.5 us and
-// 2.4 more a million partial sums (100 x 4096 -> 256 8.6 us; 256 x 3072 -> 768
-// 14.0, 512 x 2048 -> 512 12.9, 949 x 2048 -> 512 17); one launch of eight
-// waves a tile 4.2 and 0.27 a 64-deep chunk (21.0, 17.2, 12.6, 13.0).
+// Split-K when the tiles leave three quarters of the CUs idle, or any CU idle
+// with K at least 1536 deep: about two workgroups per CU, each split at least
+// 256 deep, where that is estimated to be faster.  The estimates (us; fitted on
+// an idle MI355X to 91 products of 500 .. 6000 rows, 512 .. 4096 deep, 8 ..
+// 1456 columns; 1.05 of the measured time at one standard deviation): a split
+// launch and its finishing pass 7.4, 0.35 a million partial sums written
+// (whole tiles), 1.0 a million that the pass adds (real columns) and 0.2 a
+// 32-deep chunk of each CU's share of the tiles; one launch of a tile a CU 4.2
+// and 0.27 a 64-deep chunk (eight waves) or 4.6 and 0.21 a 32-deep one (four).
+// us, split and not: 4600 x 3392 -> 24 15.5 and 18.9, 3200 x 2560 -> 24 12.3
+// and 14.9, 4500 x 3104 -> 24 14.7 and 25.4, 1100 x 2080 -> 512 16.7 and 18.7;
+// 2319 x 1664 -> 584 21.2 and 13.5, 4600 x 1536 -> 64 13.5 and 10.4, 2000 x
+// 1568 -> 512 18.3 and 15.4.  128-row tiles of few columns: not above a
+// quarter of the CUs (16500 x 1536 -> 64 20.3 split, 16.6 not).
 RowsPlan rows_plan(int cus, long workspace, int m, int k, int n, int bm, int bn, bool whole, bool split) {
   const int tiles_n = (n + bn - 1) / bn, tiles = (m + bm - 1) / bm * tiles_n, chunks = k / 32;
+  const bool eight = bm == 64 && whole && tiles <= cus && k >= 256 && k % 64 == 0;
+  const bool idle = 4 * tiles <= cus || (bm == 64 && k >= 1536 && tiles < cus);
+  if (!split || chunks < 16 || !idle) return {eight, 1};
   const long sums = (long)m * tiles_n * bn;
-  RowsPlan p{bm == 64 && whole && tiles <= cus && k >= 256 && k % 64 == 0, 1};
-  if (split && chunks >= 16 && 4 * tiles <= cus) {
-    p.ksplit = std::min(chunks / 8, (2 * cus + tiles - 1) / tiles);
-    while (p.ksplit > 1 && p.ksplit * sums > workspace) p.ksplit--;
-  }
-  if (p.eight && p.ksplit > 1) {
-    p.eight = 4.2 + 0.27 * (k / 64) < 7.5 + 2.4e-6 * p.ksplit * sums;
-    if (p.eight) p.ksplit = 1;
-  }
-  return p;
+  int ksplit = std::min(chunks / 8, (2 * cus + tiles - 1) / tiles);
+  while (ksplit > 1 && ksplit * sums > workspace) ksplit--;
+  const double one = eight ? 4.2 + 0.27 * (k / 64) : 4.6 + 0.21 * chunks;
+  const double several = 7.4 + 1e-6 * ksplit * (0.35 * sums + 1.0 * m * n) + 0.2 * tiles * chunks / cus;
+  if (ksplit == 1 || one <= several) return {eight, 1};
+  return {false, ksplit};
 }
 
 template <int BM, int BN, int KC, int MODE = 0>

@@ -81,3 +81,25 @@ def test_more_tiles_than_cus_keep_four_waves():
     assert rows_choice(CUS, WORKSPACE, 8193, 384, 256) == (4, 1)
     assert rows_choice(CUS, WORKSPACE, 64 * 257, 1536, 128) == (4, 1)
     assert rows_choice(CUS, WORKSPACE, 128 * 128, 1536, 64) == (4, 1)  # 128-row tiles
+
+
+# Deep products of few tiles: split where a tile a CU in one launch would take
+# longer (4600 x 3392 -> 24 15.5 us split, 18.9 in one; 4500 x 3104 -> 24, which
+# four waves take, 14.7 and 25.4), and in one launch where the sums cost more
+# (2319 x 1664 -> 584 13.5 us in one, 21.2 split).
+@pytest.mark.parametrize("m,k,n,want", [
+    (4600, 3392, 24, (4, 8)), (3200, 2560, 24, (4, 10)), (3256, 1728, 8, (4, 6)), (4100, 4096, 24, (4, 8)),
+    (2300, 4096, 200, (4, 8)), (4500, 3104, 24, (4, 8)), (1100, 2080, 512, (4, 8)), (100, 4096, 256, (4, 16)),
+    (2319, 1664, 584, (8, 1)), (4600, 1536, 64, (8, 1)), (4096, 1536, 384, (8, 1)), (949, 2048, 512, (8, 1)),
+    (2000, 1568, 512, (4, 1)), (16500, 1536, 64, (4, 1))])
+def test_deep_products_split_where_that_is_faster(m, k, n, want):
+    assert rows_choice(CUS, WORKSPACE, m, k, n) == want
+
+
+def test_splits_stay_in_the_workspace():
+    for m in (100, 700, 2300, 4600, 8000):
+        for k in (1536, 2560, 4096):
+            for n in (8, 64, 200, 512):
+                for workspace in (1 << 14, 1 << 20, WORKSPACE):
+                    waves, splits = rows_choice(CUS, workspace, m, k, n)
+                    assert splits == 1 or splits * m * ((n + 127) // 128 * 128) <= workspace
