@@ -24,11 +24,13 @@ def compare(ctx, x, h, w, c, n, phases, ys, act):
     import torch
 
     y = torch.full((2 * h, 2 * w, ys), 7.0, dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()  # (the library's stream need not be torch's)
     conv_up(ctx, x, h, w, c, phases, y, ys, act)
     one = torch.empty((h, w, n), dtype=torch.float16, device="cuda")
     worst = 0.0
     for p, taps in enumerate(TAPS):
         ien.multiply_ex(ctx, ien.image_input(x, h, w, c, offsets=taps), 0, h * w, phases[p], one, n, act=act)
+        torch.cuda.synchronize()
         got = y[p // 2::2, p % 2::2]
         for r in range(0, h, 256):  # (f32 copies of a band at a time)
             a, b = got[r:r + 256, :, :n].float(), one[r:r + 256].float()
@@ -36,6 +38,7 @@ def compare(ctx, x, h, w, c, n, phases, ys, act):
             # one f16 rounding (a spacing of 2^-10) either way.
             assert bool(((a - b).abs() <= 1e-5 + 2.0 ** -10 * b.abs()).all()), (p, r)
             worst = max(worst, float((a - b).abs().max()))
+        torch.cuda.synchronize()  # (`one` is read)
         assert ys == n or bool((got[..., n:] == 7.0).all())
     print(f"  {h}x{w} {c}->{n}: {worst:.3g}", flush=True)
 

@@ -67,21 +67,25 @@ def test_transforms_keep_f32_accuracy(ctx, weights, h, w):
     z = torch.empty(half * kyb * 32 * 2 * SPECTRAL, dtype=torch.float16, device="cuda")
     u = torch.empty((h, half, 2 * SPECTRAL), dtype=torch.float32, device="cuda")
     out = torch.zeros((h, w, GLOBAL), dtype=torch.float16, device="cuda")
+    flat = torch.zeros_like(spectral)
+    torch.cuda.synchronize()  # (the library's stream need not be torch's)
     sp.rows(x[..., LOCAL:], CHANNELS, m_in, spectral, r)
     sp.columns(m_f, r, z, u)
-    flat = torch.zeros_like(spectral)
     sp.back(m_out, flat, u, out, GLOBAL)
     # The f32 passes, each on the operand that the launch above read.
     f = ien.Fourier(ctx, h, w)
+    torch.cuda.synchronize()
     rows = spectral.transpose(1, 2).contiguous()
     work = torch.empty((h, half, 2 * SPECTRAL), dtype=torch.float32, device="cuda")
     spectrum = torch.empty((h, half, 2 * SPECTRAL), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
     f.forward(rows, SPECTRAL, SPECTRAL, work, spectrum)
     # z is the product's operand: [column][block of 32 rows][16 channels][half][row][8].
     zp = z.view(half, kyb, 2 * SPECTRAL // 16, 2, 32, 8).permute(0, 1, 4, 2, 3, 5)
     zp = zp.reshape(half, kyb * 32, 2 * SPECTRAL)[:, :h]
     filtered = zp.permute(1, 0, 2).clamp(min=0).contiguous()  # (the fourier matrix is the identity)
     work2, added = torch.empty_like(work), torch.zeros((h, w, SPECTRAL), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
     f.inverse(filtered, SPECTRAL, work2, added, SPECTRAL)
     torch.cuda.synchronize()
     s = spectral.double().cpu().numpy().transpose(0, 2, 1)  # [y][x][c]
@@ -146,6 +150,7 @@ def test_back_adds_to_the_map_in_place(ctx):
     d_s = torch.from_numpy(np.ascontiguousarray(s.transpose(0, 2, 1))).cuda()
     u = torch.zeros((h, half, 2 * SPECTRAL), dtype=torch.float32, device="cuda")
     d_out, d_add = torch.from_numpy(cross).cuda(), torch.from_numpy(add).cuda()
+    torch.cuda.synchronize()
     sp.back(m_out, d_s, u, d_out[..., LOCAL:], CHANNELS, d_add[..., LOCAL:], d_add[..., LOCAL:])
     torch.cuda.synchronize()
     got = d_add.cpu().numpy()
