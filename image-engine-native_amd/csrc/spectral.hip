@@ -790,7 +790,7 @@ struct TallArgs {
   const float *r;
   int h, w, half, yp, fsteps, nba, kyb;  // fsteps: 16-deep steps of F; kyb: 32-blocks of h
   float scale;  // 1 / sqrt(h w)
-  const uint16_t *ta;  // B fragments [kyb][cos | sin][bf16 piece, smallest first][fsteps]
+  const uint16_t *ta;  // B fragments [kyb][cos | sin][bf16 piece, largest first][fsteps]
   const uint16_t *tc;  // B fragments [nba][part][hi | lo][yp / 16]
   const uint16_t *wf;
   int kb_f;
@@ -800,9 +800,10 @@ struct TallArgs {
 };
 
 __global__ __launch_bounds__(512, 4) void k_spectral_tall(TallArgs p) {
-  // A fragments of the folded rows, [piece][Re | Im][E | O][step], E written
-  // by the wave that loads the step's rows of that part, O by the other's.
-  constexpr int PIECE = 4 * FOLD_STEPS * 1024;
+  // A fragments of the folded rows, [piece][Re | Im][step], first E, written by
+  // the wave that loads the step's rows of that part, then O by the other's:
+  // 24 KiB, which a CU has left beside a workgroup of the local convolution.
+  constexpr int PIECE = 2 * FOLD_STEPS * 1024;
   __shared__ __attribute__((aligned(16))) unsigned char lds[3 * PIECE];
   int k, g;
   row_part(blockIdx.x, COLUMN_GROUPS, k, g);
@@ -816,6 +817,8 @@ __global__ __launch_bounds__(512, 4) void k_spectral_tall(TallArgs p) {
   for (int q = 0; q < 3; q++)
 #pragma unroll
     for (int s = 0; s < FOLD_STEPS; s++) t[q][s] = ldb8(tb + (q * p.fsteps + min(s, p.fsteps - 1)) * 512);
+  unsigned char *to = lds + blk * 1024 + lane * 16;
+  bf16x8 o[3];
   if (blk < p.fsteps) {
     // Where R[y][m] is (m of either part; none: the imaginary parts of the
     // first and, for an even w, last column).
@@ -839,36 +842,46 @@ __global__ __launch_bounds__(512, 4) void k_spectral_tall(TallArgs p) {
       even[j] = first ? v[j] : v[j] + mirror[j];
       odd[j] = first ? mirror[j] : part ? v[j] - mirror[j] : mirror[j] - v[j];
     }
-    bf16x8 piece[3];
-    split8(even, piece);
-    unsigned char *at = lds + blk * 1024 + lane * 16;
+    bf16x8 e[3];
+    split8(even, e);
+    split8(odd, o);
 #pragma unroll
-    for (int n = 0; n < 3; n++) *(bf16x8 *)(at + n * PIECE + 2 * part * FOLD_STEPS * 1024) = piece[n];
-    split8(odd, piece);
-#pragma unroll
-    for (int n = 0; n < 3; n++) *(bf16x8 *)(at + n * PIECE + (3 - 2 * part) * FOLD_STEPS * 1024) = piece[n];
+    for (int n = 0; n < 3; n++) *(bf16x8 *)(to + n * PIECE + part * FOLD_STEPS * 1024) = e[n];
   }
   __syncthreads();
-  if (blk >= p.kyb) return;
   floatx16 acc = {}, small = {};
 #pragma unroll
-  for (int q = 0; q < 6; q++) {
-    const int piece = 2 - q % 3;  // of the table
+  for (int q = 0; q < 2; q++) {  // cos against E, sin against O
+    if (q == 1) {
+      __syncthreads();  // E is read
+      if (blk < p.fsteps) {
+#pragma unroll
+        for (int n = 0; n < 3; n++) *(bf16x8 *)(to + n * PIECE + (1 - part) * FOLD_STEPS * 1024) = o[n];
+      }
+      __syncthreads();
+    }
 #pragma unroll
     for (int s = 0; s < FOLD_STEPS; s++) {
-      if (s < p.fsteps) {
-        const unsigned char *at = lds + ((2 * part + q / 3) * FOLD_STEPS + s) * 1024 + lane * 16;
-        const bf16x8 tq = t[q % 3][s];
+      if (s < p.fsteps && blk < p.kyb) {
+        const unsigned char *at = lds + (part * FOLD_STEPS + s) * 1024 + lane * 16;
+        bf16x8 a[3];
 #pragma unroll
-        for (int n = 2 - piece; n > 0; n--) small = mfma16(*(const bf16x8 *)(at + n * PIECE), tq, small);
-        floatx16 &first = piece == 0 ? acc : small;
-        first = mfma16(*(const bf16x8 *)at, tq, first);
-        if (q < 3) t[q][s] = ldb8(tb + ((q + 3) * p.fsteps + s) * 512);
+        for (int n = 0; n < 3; n++) a[n] = *(const bf16x8 *)(at + n * PIECE);
+        acc = mfma16(a[0], t[0][s], acc);
+        small = mfma16(a[2], t[0][s], small);
+        small = mfma16(a[1], t[1][s], small);
+        small = mfma16(a[0], t[2][s], small);
+        small = mfma16(a[1], t[0][s], small);
+        small = mfma16(a[0], t[1][s], small);
+        if (q == 0) {
+#pragma unroll
+          for (int n = 0; n < 3; n++) t[n][s] = ldb8(tb + ((3 + n) * p.fsteps + s) * 512);
+        }
       }
     }
   }
   const int ky = blk * 32 + col;
-  if (ky < h) {
+  if (ky < h) {  // (blk < kyb)
     uint16_t *zb = p.z + ((long)(k * p.kyb + blk) * ZK + (part * SPEC + 32 * g) / 16) * 512 + col * 8 + 4 * hi;
 #pragma unroll
     for (int i = 0; i < 16; i++) acc[i] = (acc[i] + small[i]) * p.scale;
@@ -1306,7 +1319,7 @@ ien_status spectral_new(ien_ctx *ctx, size_t height, size_t width, ien_spectral 
     if (ky >= h || y >= (h + 1) / 2) return 0;
     const double *t = &trig_h[2 * (ky * y % h)];
     const double v = q < 3 ? t[0] : y > 0 ? t[1] : h % 2 ? 0.0 : ky % 2 ? -1.0 : 1.0;
-    return split_bf16(v, 2 - q % 3);
+    return split_bf16(v, q % 3);
   }) : operand(sp->nba, 4 * yp / 16, [&](int n, int kk) -> uint16_t {
     const int term = kk / (2 * yp), part = (kk % (2 * yp)) / yp, y = kk % yp;
     if (n >= 2 * h || y >= h) return 0;
