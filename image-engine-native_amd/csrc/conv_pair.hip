@@ -1056,11 +1056,18 @@ PairCut pair_cut(int H, int W, int cus) {
 }
 
 // A chain's tiles, smallest first.  A pair on a 16 x 24 tile takes about
-// 14 us whatever the map's size, most of it products; where smaller tiles
-// still fit the device at once, each CU has fewer of them, and LDS has room
-// for a weight buffer of its own, so that the second layer's weights land
-// behind the ring and the first layer.  The whole network on 64 x 48 pixels:
-// 229 us on 16 x 24 tiles, 127 us on 8 x 16.
+// 14 us whatever the map's size, most of it products; on smaller tiles each CU
+// has fewer of them, and LDS has room for a weight buffer of its own, so that
+// the second layer's weights land behind the ring and the first layer.  The
+// whole network on 64 x 48 pixels: 229 us on 16 x 24 tiles, 127 us on 8 x 16.
+//
+// The smaller ones only up to a quarter of the CUs: a process runs kernels of
+// up to 4 streams at once, and as many chains of small maps, each waiting for
+// tiles of its own, have to fit side by side, as they did on 16 x 24 tiles.
+// (With up to a tile a CU two contexts on 128 x 256 pixels, 88 tiles of 16 x 24
+// or 256 of 8 x 16, now and then started together, kept CUs from each other and
+// gave up waiting: once in 3000 runs.)  Maps over some 12000 pixels stay on
+// 16 x 24 tiles: 128 x 128 pixels 221 us, where 128 tiles of 8 x 16 took 141.
 using SmallTile = Geo<8, 16, true>;
 using MiddleTile = Geo<12, 16, true>;
 using LargeTile = Geo<16, 24, false>;
@@ -1078,12 +1085,22 @@ long tile_count(const ChainTile &t, int H, int W) {
   return (long)((W + t.cols - 1) / t.cols) * ((H + t.rows - 1) / t.rows);
 }
 
+}  // namespace
+
+int chain_choice(int cus, int H, int W) {
+  constexpr int LAST = ien_ctx::CHAIN_TILINGS - 1;
+  for (int i = 0; i < LAST; i++)
+    if (4 * tile_count(CHAIN_TILES[i], H, W) <= cus) return i;
+  return tile_count(CHAIN_TILES[LAST], H, W) <= cus ? LAST : -1;
+}
+
+namespace {
+
 // The smallest tiling of a map whose workgroups are all resident at once
 // (one per CU at most), or null.
 const ChainTile *chain_tile(ien_ctx *ctx, int H, int W) {
-  for (int i = 0; i < ien_ctx::CHAIN_TILINGS; i++) {
-    const long tiles = tile_count(CHAIN_TILES[i], H, W);
-    if (tiles > (long)ctx->cus || tiles > ctx->chain_tiles) continue;
+  for (int i = chain_choice(ctx->cus, H, W); i >= 0 && i < ien_ctx::CHAIN_TILINGS; i++) {
+    if (tile_count(CHAIN_TILES[i], H, W) > ctx->chain_tiles) continue;
     int &per_cu = ctx->chain_per_cu[i];
     if (per_cu < 0) {
       int n = 0;

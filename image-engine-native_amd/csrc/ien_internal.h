@@ -292,6 +292,9 @@ struct ChainCall {
   const float *first_slope = nullptr;
 };
 bool chain_supported(ien_ctx *ctx, const ChainCall &c);
+// The chain's tiling of an H x W map on a device of `cus` CUs: 8 x 16, 12 x 16
+// or 16 x 24 tiles (0, 1, 2), or -1 where the device does not hold them.
+int chain_choice(int cus, int H, int W);
 ien_status launch_chain(ien_ctx *ctx, const ChainCall &c, uint16_t **out);
 ien_status chain_status(ien_ctx *ctx, int first);
 

@@ -78,3 +78,9 @@ def rows_choice(cus, workspace, m, k, n):
     """conv_common.h rows_choice: (waves a tile, splits)."""
     r = _function("_ZN3ien11rows_choiceEiliii", _int, _long, _int, _int, _int)(cus, workspace, m, k, n)
     return 8 if r < 0 else 4, abs(r)
+
+
+def chain_choice(cus, h, w):
+    """ien_internal.h chain_choice: the rows and columns of a chain's tiles, or None."""
+    i = _function("_ZN3ien12chain_choiceEiii", _int, _int, _int)(cus, h, w)
+    return None if i < 0 else [(8, 16), (12, 16), (16, 24)][i]

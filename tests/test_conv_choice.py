@@ -1,9 +1,9 @@
-"""The sizes that the convolution and row-product kernels accept, and which of
-them a size takes (host code, no GPU)."""
+"""The sizes that the convolution, chain and row-product kernels accept, and
+which of them a size takes (host code, no GPU)."""
 
 import pytest
 
-from internal import conv3_choice, conv_up_fits, rows_choice, stride2_choice
+from internal import chain_choice, conv3_choice, conv_up_fits, rows_choice, stride2_choice
 
 CUS, WORKSPACE = 256, 8 << 20  # MI355X; the context's workspace in floats
 
@@ -103,3 +103,27 @@ def test_splits_stay_in_the_workspace():
                 for workspace in (1 << 14, 1 << 20, WORKSPACE):
                     waves, splits = rows_choice(CUS, workspace, m, k, n)
                     assert splits == 1 or splits * m * ((n + 127) // 128 * 128) <= workspace
+
+
+# A chain's workgroups wait for each other, so all of them have to be resident:
+# the chains of small maps on smaller tiles take a quarter of the CUs at most,
+# so that the four streams that a process runs at once hold one each, as they
+# did on 16 x 24 tiles.
+@pytest.mark.parametrize("h,w,want", [
+    (1, 1, (8, 16)), (48, 64, (8, 16)), (64, 128, (8, 16)), (65, 128, (12, 16)), (72, 160, (12, 16)),
+    (96, 128, (12, 16)), (97, 128, (16, 24)), (128, 128, (16, 24)), (128, 256, (16, 24)), (192, 256, (16, 24)),
+    (256, 384, (16, 24)), (257, 384, None), (256, 385, None), (8, 1024, (8, 16)), (8, 1025, (16, 24))])
+def test_chain_tilings(h, w, want):
+    assert chain_choice(CUS, h, w) == want
+
+
+def test_four_chains_that_fitted_on_large_tiles_fit():
+    for h in range(1, 400, 3):
+        for w in range(1, 500, 7):
+            large = ((h + 15) // 16) * ((w + 23) // 24)
+            tile = chain_choice(CUS, h, w)
+            assert (tile is None) == (large > CUS)
+            if tile:
+                tiles = -(-h // tile[0]) * -(-w // tile[1])
+                for streams in (1, 2, 3, 4):
+                    assert streams * large > CUS or streams * tiles <= CUS

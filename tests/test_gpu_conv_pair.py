@@ -1,8 +1,8 @@
 """GPU: the body kernels' tilings give the bits of single-layer launches.
 
 ien_conv3_pair cuts a map into strips of 62 or 30 columns by segments of
-rows, ien_conv3_chain into 8 x 16, 12 x 16 or 16 x 24 tiles by how many the
-device holds at once (256 CUs).  Both are compared, bit for bit, with one
+rows, ien_conv3_chain into 8 x 16 or 12 x 16 tiles where they take at most a
+quarter of the 256 CUs and else into 16 x 24 tiles, a CU each at most.  Both are compared, bit for bit, with one
 ien_conv3 launch per layer at the edges of those cuts."""
 
 import numpy as np
@@ -61,11 +61,12 @@ def test_pair_strips(ctx, layers, h, w):
     assert same_bits(y, single(ctx, x, h, w, layers[:2]))
 
 
-# Both sides of each tiling's 256 tiles (8 x 16 up to 128 x 256 pixels,
-# 12 x 16 up to 192 x 256, 16 x 24), partial tiles on both edges, last tiles
-# narrower than the 2-pixel border.
+# Both sides of the smaller tilings' 64 tiles (8 x 16 up to 64 x 128 pixels,
+# 12 x 16 up to 96 x 128) and of 256 tiles of 16 x 24, partial tiles on both
+# edges, last tiles narrower than the 2-pixel border.
 @pytest.mark.parametrize("h,w", [(1, 1), (9, 17), (7, 100), (128, 256), (129, 256), (121, 273), (192, 256),
-                                 (193, 256), (181, 273), (256, 384), (241, 361)])
+                                 (193, 256), (181, 273), (256, 384), (241, 361), (64, 128), (65, 128), (57, 113),
+                                 (96, 128), (97, 128), (85, 113), (61, 161), (8, 1009), (1, 1025)])
 def test_chain_tilings(ctx, layers, h, w):
     import ien
     import torch
