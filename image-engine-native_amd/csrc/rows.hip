@@ -25,15 +25,15 @@
 //    gemm.rs:583-666.
 // Chunks of 32 channels keep the ring at 36 KiB (64 x 128 tiles), so several
 // workgroups share a CU and hide each other's latency.
-// Where the tiles leave no CU a second workgroup (KG = 2; rows_plan) nothing hides the
-// latency of four waves that wait for a chunk, read its fragments and
-// multiply them in turn (a 32-deep chunk took some 0.18 us, 0.05 of them
+// Where the tiles leave no CU a second workgroup (KG = 2; rows_plan) nothing
+// hides the latency of four waves that wait for a chunk, read its fragments
+// and multiply them in turn (a 32-deep chunk took some 0.18 us, 0.05 of them
 // products).  There eight waves take a tile: chunks are 64 deep, each set of
 // four waves takes half of a chunk's steps, a chunk's fragments are read while
 // the one before is multiplied, and the two sets' sums meet in the epilogue's
 // LDS.  us, four waves (with their split-K) -> eight: 4096 x 1536 -> 384
-// 22.5 -> 11.6, 3269 x 1536 -> 384 19.5 -> 11.5, 1024 x 384 -> 384 7.8 -> 5.9,
-// 949 x 2048 -> 512 16.8 -> 13.0.  Over a CU's worth of tiles the four waves
+// 21.8 -> 11.2, 3269 x 1536 -> 384 19.0 -> 11.3, 1024 x 384 -> 384 7.3 -> 5.6,
+// 949 x 2048 -> 512 16.2 -> 13.0.  Over a CU's worth of tiles the four waves
 // stay the faster ones (24576 x 128 -> 512 16.7 against 20.5).
 // Tiles are dealt XCD-aware with N fastest, so a tile row's x stays in its
 // XCD's L2 for every column tile.
@@ -421,11 +421,13 @@ struct RowsPlan {
 };
 
 // Eight waves a tile where a CU gets at most one of them (see above), in 64-deep
-// chunks (`whole`: each lies in one plane or pixel) and with four of them or
-// more: below that four waves, several tiles a CU, are the faster ones (us,
-// four waves -> eight: 3951 x 64 -> 192 4.2 -> 4.7, 8000 x 192 -> 256 5.5 ->
-// 6.0, 900 x 128 -> 128 4.5 -> 4.6; 1762 x 256 -> 520 5.7 -> 5.5, 8000 x 384
-// -> 256 7.0 -> 6.5).
+// chunks (`whole`: each lies in one plane or pixel).  Of fewer than four chunks
+// only under 96 tiles: over that four waves are the faster ones (us, four waves
+// -> eight: 3951 x 64 -> 192 4.2 -> 4.7, 8000 x 192 -> 256 5.5 -> 6.0; 1762 x
+// 256 -> 520 5.7 -> 5.5, 8000 x 384 -> 256 7.0 -> 6.5); under it they are level
+// on operands that the L2 holds (900 x 128 -> 128 4.5 and 4.6), and on those
+// that it does not all chunks of eight waves are in flight at once (a whole
+// SCUNet of 128 x 256 pixels 1346 -> 1317).
 //
 // Split-K when the tiles leave three quarters of the CUs idle, or any CU idle
 // with K at least 1536 deep: about two workgroups per CU, each split at least
@@ -443,7 +445,7 @@ struct RowsPlan {
 // quarter of the CUs (16500 x 1536 -> 64 20.3 split, 16.6 not).
 RowsPlan rows_plan(int cus, long workspace, int m, int k, int n, int bm, int bn, bool whole, bool split) {
   const int tiles_n = (n + bn - 1) / bn, tiles = (m + bm - 1) / bm * tiles_n, chunks = k / 32;
-  const bool eight = bm == 64 && whole && tiles <= cus && k >= 256 && k % 64 == 0;
+  const bool eight = bm == 64 && whole && tiles <= cus && (k >= 256 || tiles < 96) && k % 64 == 0;
   const bool idle = 4 * tiles <= cus || (bm == 64 && k >= 1536 && tiles < cus);
   if (!split || chunks < 16 || !idle) return {eight, 1};
   const long sums = (long)m * tiles_n * bn;
@@ -491,10 +493,10 @@ ien_status launch(ien_ctx *ctx, RowsArgs a, const ConvArgs &c) {
 static long tiles_of(long rows, int bm, int n) { return (rows + bm - 1) / bm * ((n + 127) / 128); }
 
 // Any number of tiles of 64s of channels (104 x 384 -> 384 7.4 us on the
-// general kernel, 5.8 here; 145 x 1024 -> 256 10.4 and 8.4; 900 x 128 -> 128
-// 5.4 and 4.5); else 128-row tiles when they number
-// at least 128, 64-row tiles when those number at least 96, or at least 8
-// with K 512 deep (split-K); below that the general kernel serves.
+// general kernel, 5.4 here; 145 x 1024 -> 256 10.3 and 7.6; 900 x 128 -> 128
+// 5.3 and 4.4); else 128-row tiles when they number at least 128, 64-row
+// tiles when those number at least 96, or at least 8 with K 512 deep
+// (split-K); below that the general kernel serves.
 bool rows_supported(const ConvArgs &a, long rows) {
   const bool aligned = (((uintptr_t)a.x) & 15) == 0 && (((uintptr_t)a.y) & 15) == 0;
   const long t64 = tiles_of(rows, 64, a.N);

@@ -65,16 +65,23 @@ def test_stride2_bands_choose_by_their_own_rows():
     assert stride2_choice(CUS, 256, 64, 2 * 256, 130 * 256) == 16
 
 
-# Products of few channels keep four waves a tile: eight, which wait for no
-# other workgroup, lose on three 64-deep chunks and less (3951 x 64 -> 192 4.2
-# us on four, 4.7 on eight).
-@pytest.mark.parametrize("m,n", [(1, 8), (900, 128), (1762, 520), (3951, 192), (8000, 256), (8192, 256)])
+# Products of few channels and 96 tiles or more keep four waves a tile: eight
+# lose on three 64-deep chunks and less (3951 x 64 -> 192 4.2 us on four, 4.7 on
+# eight).
+@pytest.mark.parametrize("m,n", [(96 * 64, 128), (1762, 520), (3951, 192), (8000, 256), (8192, 256)])
 def test_shallow_products_keep_four_waves(m, n):
     for k in (64, 128, 192):
         assert rows_choice(CUS, WORKSPACE, m, k, n) == (4, 1)
     for k in (256, 384, 448):
         assert rows_choice(CUS, WORKSPACE, m, k, n) == (8, 1)
     assert rows_choice(CUS, WORKSPACE, m, 288, n) == (4, 1)  # (not whole 64-deep chunks)
+
+
+@pytest.mark.parametrize("m,n", [(1, 8), (900, 128), (95 * 64, 128)])
+def test_shallow_products_of_few_tiles_take_eight_waves(m, n):
+    for k in (64, 128, 192, 256):
+        assert rows_choice(CUS, WORKSPACE, m, k, n) == (8, 1)
+    assert rows_choice(CUS, WORKSPACE, m, 96, n) == (4, 1)
 
 
 def test_more_tiles_than_cus_keep_four_waves():

@@ -493,11 +493,11 @@ def test_rows_tiles(ctx, oracle, m, k, n, act, acc, row0, pad):
     close(got[:, :n], want)
 
 
-# Eight waves a tile (at most a CU's worth of 64 x 128 tiles, K in 64s from
-# 256): one row, rows and columns about a tile's edge, an odd count of chunks
-# (which ends with a step of zeros) and an even one, exactly 256 tiles, and
-# split where K is deep; shallow products and one row more than 256 tiles
-# beside them, on four waves.
+# Eight waves a tile (at most a CU's worth of 64 x 128 tiles, K in 64s, from 256
+# where they are 96 or more): one row, rows and columns about a tile's edge, one
+# chunk (an odd count ends with a step of zeros) to deep ones, exactly 256 tiles,
+# and split where K is deep; a shallow product of 256 tiles and one row more than
+# 256 tiles beside them, on four waves.
 @pytest.mark.parametrize("m,k,n,act,acc,row0,pad", [
     (1, 64, 8, 0, False, 0, 0), (63, 128, 136, 1, True, 3, 8), (65, 192, 128, 2, False, 0, 0),
     (64, 320, 120, 3, True, 0, 8), (500, 1536, 392, 0, True, 0, 0), (8192, 192, 256, 2, False, 0, 0),
