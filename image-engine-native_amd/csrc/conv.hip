@@ -1213,10 +1213,11 @@ static int pick_ck(int c) { return c % 64 == 0 ? 64 : c % 32 == 0 ? 32 : 16; }
 // Microseconds that an NHWC 3 x 3 stride-1 product of 64s of channels takes
 // here, by the number of its 4 x 32 x 64 tiles: one round of double-buffered
 // workgroups (with their splits), two a CU on 16-channel chunks, or
-// single-buffered ones.  Fitted to sweeps on an idle MI355X (us, measured:
-// 64 x 96, 256 -> 256 14.5; 85 x 125, 512 -> 128 25.5; 128 x 192, 128 -> 128
-// 12.8; 95 x 95, 512 -> 256 34; 85 x 125, 128 -> 384 19.7; 71 x 472,
-// 512 -> 128 65; 200 x 200, 256 -> 256 70).
+// single-buffered ones.  Fitted to sweeps on an idle MI355X (us, estimated and
+// as measured on one box since: 64 x 96, 256 -> 256 15.1 and 15.0; 85 x 125,
+// 512 -> 128 24.7 and 23.0; 128 x 192, 128 -> 128 12.8 and 13.2; 95 x 95, 512 ->
+// 256 35.0 and 32.3; 85 x 125, 128 -> 384 19.7 and 19.1; 71 x 472, 512 -> 128
+// 65 and 60; 200 x 200, 256 -> 256 70 and 66).
 static double general_us(int cus, int ow, int c, int n, long p_begin, long p_end) {
   const long tiles = range_tiles(ow, p_begin, p_end, n, 4, 64);
   const int chunks = c / 32;
@@ -1237,9 +1238,9 @@ int conv3_choice(int cus, long workspace, int ow, int c, int n, long p_begin, lo
 // 32-channel chunks where a CU gets at most one tile of the range
 // (double-buffered: 128 x 128, 256 -> 512 19.1 us, 21.6 with 16); over that
 // 16-channel ones, whose halo and weights leave room for four workgroups a CU
-// instead of two (us, 32 -> 16: 680 x 1000, 64 -> 128 69.6 -> 57.6; 340 x 500,
-// 128 -> 256 60.7 -> 54.7; 170 x 250, 256 -> 512 74.9 -> 54.9; 512 x 512,
-// 64 -> 128 26.7 -> 24.4).
+// instead of two (us, 32 -> 16: 680 x 1000, 64 -> 128 67.8 -> 51.0; 340 x 500,
+// 128 -> 256 57.7 -> 49.1; 170 x 250, 256 -> 512 66.3 -> 47.3; 512 x 512,
+// 64 -> 128 26.4 -> 22.8).
 int stride2_choice(int cus, int ow, int n, long p_begin, long p_end) {
   return range_tiles(ow, p_begin, p_end, n, 4, 64) <= cus ? 32 : 16;
 }

@@ -394,10 +394,10 @@ struct Tile {
 // tap order.  No row is computed twice within a segment.
 //
 // Bound by the matrix cores: 836 x 836 pixels (103 GFLOP a pair) take 96 us
-// a pair, MFMA busy 73 % of a workgroup's life, the rest of the launch its
-// start and drain.  16 x 24 tiles, which stage 144 KiB of weights and wait
-// for them and for the halo once a tile, took 130 us there (the whole
-// network 2.27 -> 1.67 ms); 12 x 16 tiles with every load overlapped 142.
+// a pair, MFMA busy 59 % of the device's SIMD cycles over the launch, its
+// start and drain included.  16 x 24 tiles, which stage 144 KiB of weights and
+// wait for them and for the halo once a tile, took 130 us there (the whole
+// network 2.28 -> 1.64 ms); 12 x 16 tiles with every load overlapped 142.
 // B fragments 1, 2, 3, 4 products ahead: 1725, 1655, 1647, 1647 us.
 template <int R>
 struct Strip {

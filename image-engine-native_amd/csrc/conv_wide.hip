@@ -366,14 +366,16 @@ constexpr double SPLIT_US = 6.0;
 }  // namespace
 
 // Whole 16-byte groups of f16 NHWC outputs, ranges in 31 bits.  Measured
-// against the general kernel on an idle MI355X (us, general -> here):
-// 85 x 125, 512 -> 128 26.2 -> 19.8 (4 x 64 tiles; 22.9 as 4 x 128 in 2
-// splits) and 128 -> 384 19.7 -> 17.9 (8 x 128); 64 x 96, 256 -> 256
-// 14.9 -> 12.8 and 64 x 64, 128 -> 384 10.7 -> 9.2 (4 x 64); 71 x 472,
-// 512 -> 128 65 -> 48 (8 x 128); 200 x 200, 256 -> 256 70 -> 56; 95 x 95,
-// 512 -> 256 34 -> 28 (8 x 64); and, left to the general kernel's deep
-// splits, 64 x 64, 512 -> 128 14.4 against 17.9.  Not compact launches: a workgroup leaves
-// another branch's kernels no LDS.
+// against the general kernel on one idle MI355X (us, general -> here; the same
+// shape moves by some 3 % from box to box): 85 x 125, 512 -> 128 23.0 -> 19.2
+// (4 x 64 tiles; 22.9 as 4 x 128 in 2 splits) and 128 -> 384 19.1 -> 18.3
+// (8 x 128); 64 x 96, 256 -> 256 15.0 -> 12.8 and 64 x 64, 128 -> 384 10.1 ->
+// 9.3 (4 x 64); 71 x 472, 512 -> 128 60 -> 49 (8 x 128); 200 x 200, 256 -> 256
+// 66 -> 63; 95 x 95, 512 -> 256 32 -> 29; and, left to the general kernel's
+// deep splits, 64 x 64, 512 -> 128 14.4 against 17.9.  Over 215 sizes of 1 ..
+// 400 rows and 4 .. 400 columns, 64 .. 1024 -> 64 .. 512 channels, the choice
+// took 0.95 of the general kernel's time in the mean, at worst 1.02 of it.  Not
+// compact launches: a workgroup leaves another branch's kernels no LDS.
 bool wide_supported(const ien_ctx *ctx, const ConvArgs &a) {
   return a.C % 64 == 0 && a.N % 8 == 0 && a.ys % 8 == 0 && (((uintptr_t)a.y | (uintptr_t)a.add2) & 15) == 0 &&
          !a.out_nchw && !a.out_f32 && !ctx->compact && (long)a.H * a.W * a.xs * 2 <= 0x7fff0000L &&
@@ -414,8 +416,8 @@ bool conv_up_fits(long h, long w, long c, long n, long ys) {
 }
 
 // LaMa's doublings (1000 x 680 images, us): 85 x 125, 512 -> 256 as four
-// launches of the general kernel 112, here 43; 170 x 250, 256 -> 128 112 and
-// 48; 340 x 500, 128 -> 64 110 and 57.
+// launches of the general kernel 108, here 37; 170 x 250, 256 -> 128 109 and
+// 48; 340 x 500, 128 -> 64 107 and 62.
 ien_status conv_up(ien_ctx *ctx, const uint16_t *x, int h, int w, int c, ien_matrix *const *phases, uint16_t *y,
                    int ys, ien_act act) {
   const int n = (int)phases[0]->n;

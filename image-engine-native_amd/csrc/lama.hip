@@ -226,8 +226,8 @@ ien_status lama_reserve(Lama *l, size_t pw, size_t ph, bool *grew) {
     ien_spectral_free(l->spectral_plan);
     l->spectral_plan = nullptr;
     // The fused spectral branch takes maps of sides up to 128 (images up to
-    // 1024 x 1024: 1000 x 680 ran in 6.21 ms on the unfused chain, 4.07 ms on
-    // the fused one); larger ones run the unfused chain.
+    // 1024 x 1024: alone it took 1000 x 680 ones from 6.21 to 4.07 ms);
+    // larger ones run the unfused chain.
     const ien_status st = spectral_fits(h8, w8) ? spectral_new(l->ctx, h8, w8, &l->spectral_plan)
                                                 : ien_fourier_new(l->ctx, h8, w8, &l->fourier);
     if (st != IEN_OK) return st;
@@ -266,25 +266,6 @@ ien_status lama_reserve(Lama *l, size_t pw, size_t ph, bool *grew) {
   return IEN_OK;
 }
 
-// network.rs:415-489 Network::run.
-// The 18 blocks' FFCs with the fused spectral branch (network.rs:249-262,
-// x += ffc1(ffc0(x)): the second FFC's local convolution and back launch
-// add their rounded results onto x in place, the sums ien_add would make),
-// as a pipeline over three streams.  FFC k: its spectral rows (192 short
-// workgroups) and then its local convolution on the context's stream (the
-// local convolution enqueued before the branches' launches, so that its
-// workgroups, one a CU, are not held back behind theirs), its spectral
-// columns on branch 1, its back launch on the context's stream after both
-// (R in the spectrum buffer, a tall map's spectrum in the filtered buffer, U
-// in the work buffer).  Its cross
-// convolution reads only the local part of its input, which the previous
-// FFC's local convolution has written: it runs on branch 2 from there on,
-// beside that FFC's columns and back launch (which leave CUs idle: 192
-// workgroups of one a CU each).  What the early cross convolution writes
-// (the global part of FFC k's output map) no launch before FFC k's back
-// reads: FFC k - 1 reads the other map (or, for the second FFC of a
-// block, x, whose global part it only reads in its rows and local launches,
-// both before the wait).
 struct Serial {  // every branch on the context's stream while it lives
   ien_ctx *ctx;
   bool was;
@@ -294,6 +275,23 @@ struct Serial {  // every branch on the context's stream while it lives
   Serial &operator=(const Serial &) = delete;
 };
 
+// The 18 blocks' FFCs with the fused spectral branch (network.rs:249-262,
+// x += ffc1(ffc0(x)): the second FFC's local convolution and back launch
+// add their rounded results onto x in place, the sums ien_add would make),
+// as a pipeline over three streams.  FFC k: its spectral rows (192 short
+// workgroups) and then its local convolution on the context's stream (the
+// local convolution enqueued before the branches' launches, so that its
+// workgroups, one a CU, are not held back behind theirs), its spectral
+// columns on branch 1, its back launch on the context's stream after both
+// (R in the spectrum buffer, the spectrum of a map with a side over 64 in the
+// filtered buffer, U in the work buffer).  Its cross convolution reads only the local part of its input, which the previous
+// FFC's local convolution has written: it runs on branch 2 from there on,
+// beside that FFC's columns and back launch (which leave CUs idle: 192
+// workgroups of one a CU each).  What the early cross convolution writes
+// (the global part of FFC k's output map) no launch before FFC k's back
+// reads: FFC k - 1 reads the other map (or, for the second FFC of a
+// block, x, whose global part it only reads in its rows and local launches,
+// both before the wait).
 template <class Done>
 ien_status ffc_pipeline(Lama *l, int h, int w, Done &done) {
   ien_ctx *ctx = l->ctx;
@@ -375,6 +373,7 @@ ien_status ffc_pipeline(Lama *l, int h, int w, Done &done) {
   return st;
 }
 
+// network.rs:415-489 Network::run.
 ien_status lama_enqueue(Lama *l, const float *d_image, const float *d_mask, size_t width,
                         size_t height, float *d_out, Steps *steps) {
   ien_ctx *ctx = l->ctx;

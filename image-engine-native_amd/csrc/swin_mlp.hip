@@ -137,8 +137,9 @@ __global__ __launch_bounds__(256) void k_swin_mlp(MlpArgs a) {
     for (int s = 0; s < S::KS1; s++) w1f[s] = *(const half8 *)(w1 + s * 512);
     // The units are the product's rows (the weights its A operand), so that a
     // lane holds four consecutive units of one token: 8-byte writes, and the
-    // bias is where the sums start (us a block, with one product less in
-    // gelu_f: 96 channels at 256 x 256 104.7 -> 102, 64 at 256 x 384 57.3 -> 56.4).
+    // bias is where the sums start (us a block and a copy of its map, with one
+    // product less in gelu_f: 96 channels at 256 x 256 104.7 -> 102, 64 at 256 x
+    // 384 57.3 -> 56.4).
     floatx16 h0, h1;
     const float *b1 = a.b1 + ch * MLP_CHUNK + wave * 32 + 4 * hf;
 #pragma unroll
@@ -240,10 +241,11 @@ __global__ __launch_bounds__(256) void k_swin_mlp(MlpArgs a) {
 // over the units in that order, on both operands.  One lane swap at the end
 // brings the output to the order of the rows as they were loaded, so the
 // residual comes from registers.
-// Measured on a 256 x 256 map of 96 channels (windows of 12, us a block): 102
+// Measured on a 256 x 256 map of 96 channels (windows of 12, us a block): 95.9
 // with the chunks above, whose 1024 workgroups each load the weights again and
-// wait at a barrier a chunk, 83 here.  What bounds it is VALU work: 22 issue
-// slots a GELU, 12.6 M values a CU's lanes at a time, some 14 us of it.
+// wait at a barrier a chunk, 74.6 here.  What bounds it is VALU work: a GELU is
+// 19 instructions, one of them a reciprocal at a quarter of the rate, so 22
+// issue slots, and 25.2 M of them make some 14 us.
 template <int C>
 struct Strip {
   static constexpr int KS1 = C / 16, UB = C / 8, CB = C / 32, KS2 = C / 4;
