@@ -11,7 +11,7 @@ input already resident in HBM: a step is one launch, the whole network as
 one chain (ien_model_run_device with graphs on: a run of one launch is
 launched directly).  Prints one JSON line.
 
-roofline: the dominant kernel is that launch, conv_pair<chain>: the first
+roofline: the dominant kernel is that launch, conv_chain: the first
 layer (3 -> 64), the 32 body layers (3x3 64->64 + PReLU each, 16 pairs)
 and the last layer (64 -> 48) plus the pixel shuffle and the image added.
 Its algorithmic work per launch is 2 * 98304 px * 576 * 64 * 32 (body)
@@ -850,7 +850,7 @@ def main():
     roofline = {"bound": "mfma", "achieved": round(achieved, 1), "peak": MFMA_F16_PEAK_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(achieved / MFMA_F16_PEAK_TFLOPS, 4),
                 "traffic": traffic_from_profiles(),
-                "kernel": "conv_pair<chain> (the whole network in one launch: first layer, 32 body "
+                "kernel": "conv_chain (the whole network in one launch: first layer, 32 body "
                           "layers 3x3 64->64 + PReLU, last layer + pixel shuffle, 256x384)",
                 "kernel_us": round(kms * 1e3, 2), "flop_per_launch": flops,
                 "rocprof": counters_from_profiles("esrgan")}
